@@ -8,10 +8,8 @@
 // GELU/ReLU, residual add into the fp32 stream, RoPE on q/k, GEGLU -- works on
 // the accumulators in registers, and the tile order is XCD-aware.
 //
-// Generic path (any shape, fp32 or bf16): 64x64x16 LDS tiles with 4x4 FMA
-// micro-tiles per thread and the same LDS-staged epilogue.  It serves the fp32
-// parity mode and the shapes the MFMA tiling does not cover (tiny models, the
-// scorer's N = 1 projection, LoRA ranks).
+// The fp32 parity mode and the shapes the bf16 tiling does not cover (tiny
+// models, the scorer's N = 1 projection, LoRA ranks) go to gemm_f32.hip.
 #include <algorithm>
 #include <type_traits>
 
@@ -22,78 +20,6 @@
 namespace sjh {
 
 namespace {
-
-// ---- epilogue over an fp32 BMxBN tile staged in LDS (row stride ldcs) ----
-template <int BM, int BN, int NT, typename OutT>
-__device__ __forceinline__ void tile_epilogue(const float* Cs, int ldcs, int m0, int tile_n,
-                                              const GemmArgs g) {
-  const int tid = threadIdx.x;
-  if (g.epi == EPI_GEGLU) {
-    constexpr int HB = BN / 2;
-    const int j0 = tile_n * HB;
-    OutT* out = static_cast<OutT*>(g.out);
-    for (int idx = tid; idx < BM * HB; idx += NT) {
-      const int r = idx / HB, c = idx - r * HB;
-      const int m = m0 + r, j = j0 + c;
-      if (m < g.M && j < g.N) {
-        const float in = Cs[r * ldcs + c], gate = Cs[r * ldcs + HB + c];
-        store_f32(out + static_cast<int64_t>(m) * g.ldo + j, gelu_out<OutT>(in) * gate);
-      }
-    }
-    return;
-  }
-  const int n0 = tile_n * BN;
-  for (int idx = tid; idx < BM * BN; idx += NT) {
-    const int r = idx / BN, c = idx - r * BN;
-    const int m = m0 + r, n = n0 + c;
-    if (m >= g.M || n >= g.N) continue;
-    float v = Cs[r * ldcs + c];
-    if (g.epi == EPI_RESID) {
-      if (g.bias) v += g.bias[n];
-      g.X[static_cast<int64_t>(m) * g.ldx + n] += v;
-      continue;
-    }
-    if (g.epi == EPI_ROPE) {
-      if (n < 2 * g.rope_dim) {
-        const int hd = g.head_dim, half = hd >> 1;
-        const int dd = n % hd;
-        const int64_t p = min(max(g.pos[m], 0), g.rope_rows - 1);
-        if (dd < half) {
-          const float x1 = Cs[r * ldcs + c + half];
-          const float cs = g.rope_cos[p * half + dd], sn = g.rope_sin[p * half + dd];
-          v = rope_lo(v, x1, cs, sn);
-        } else {
-          const int d2 = dd - half;
-          const float x0 = Cs[r * ldcs + c - half];
-          const float cs = g.rope_cos[p * half + d2], sn = g.rope_sin[p * half + d2];
-          v = rope_hi(x0, v, cs, sn);
-        }
-        if (n < g.rope_dim) v *= g.q_scale;
-      }
-    } else {
-      if (g.bias) v += g.bias[n];
-      if (g.act == 1)
-        v = gelu_out<OutT>(v);
-      else if (g.act == 2)
-        v = fmaxf(v, 0.f);
-    }
-    store_f32(static_cast<OutT*>(g.out) + static_cast<int64_t>(m) * g.ldo + n, v);
-  }
-}
-
-// W row feeding tile row i of column tile tile_n (GEGLU: first half of the
-// tile = input rows, second half = gate rows of the reference's [2F, K] Wi).
-template <int BN>
-__device__ __forceinline__ int64_t w_row(const GemmArgs g, int tile_n, int i) {
-  if (g.epi == EPI_GEGLU) {
-    constexpr int HB = BN / 2;
-    const int j = tile_n * HB + (i < HB ? i : i - HB);
-    const int jc = j < g.N ? j : g.N - 1;
-    return i < HB ? jc : static_cast<int64_t>(g.N) + jc;
-  }
-  const int n = tile_n * BN + i;
-  return n < g.N ? n : g.N - 1;
-}
 
 // ------------------------------------------------------------------ MFMA bf16
 //
@@ -2078,81 +2004,6 @@ bool launch_splitk(const GemmArgs& g0, hipStream_t st) {
   return true;
 }
 
-// ------------------------------------------------------------------ generic
-constexpr int gBM = 64, gBN = 64, gBK = 16;
-constexpr int gLdc = gBN + 4;
-
-template <typename InT, typename OutT>
-__global__ __launch_bounds__(256) void gemm_generic_kernel(GemmArgs g0) {
-  const GemmArgs g = resolve_rows(g0);
-  constexpr int kStage = 2 * gBK * (gBM + 1);  // As[k][m] and Ws[k][n]
-  constexpr int kFloats = kStage > gBM * gLdc ? kStage : gBM * gLdc;
-  __shared__ float smem[kFloats];
-  float* As = smem;
-  float* Ws = smem + gBK * (gBM + 1);
-
-  const int tile_n = blockIdx.x, tile_m = blockIdx.y;
-  const int m0 = tile_m * gBM;
-  if (m0 >= g.M) return;  // uniform
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const InT* A = static_cast<const InT*>(g.A);
-  const InT* W = static_cast<const InT*>(g.W);
-
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-  for (int k0 = 0; k0 < g.K; k0 += gBK) {
-    // 64 rows x 16 k per operand: 1024 elements, 4 per thread
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i, row = c >> 4, kk = c & 15;
-      const int k = k0 + kk;
-      const int m = m0 + row;
-      float av = 0.f, wv = 0.f;
-      if (k < g.K) {
-        if (m < g.M) av = load_f32(A + static_cast<int64_t>(m) * g.lda + k);
-        wv = load_f32(W + w_row<gBN>(g, tile_n, row) * g.ldw + k);
-      }
-      As[kk * (gBM + 1) + row] = av;
-      Ws[kk * (gBN + 1) + row] = wv;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < gBK; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk * (gBM + 1) + ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Ws[kk * (gBN + 1) + tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-    }
-    __syncthreads();
-  }
-  float* Cs = smem;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) Cs[(ty * 4 + i) * gLdc + tx * 4 + j] = acc[i][j];
-  __syncthreads();
-  tile_epilogue<gBM, gBN, 256, OutT>(Cs, gLdc, m0, tile_n, g);
-}
-
-template <typename InT>
-void launch_generic(const GemmArgs& g, hipStream_t st) {
-  const int ntiles = g.epi == EPI_GEGLU ? (g.N + gBN / 2 - 1) / (gBN / 2) : (g.N + gBN - 1) / gBN;
-  dim3 grid(ntiles, (g.M + gBM - 1) / gBM), block(256);
-  if (g.out_dtype == DT_BF16)
-    gemm_generic_kernel<InT, bf16_t><<<grid, block, 0, st>>>(g);
-  else
-    gemm_generic_kernel<InT, float><<<grid, block, 0, st>>>(g);
-}
-
 }  // namespace
 
 // The bf16 MFMA kernels' operand requirements.
@@ -2252,7 +2103,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
                     (g.epi != EPI_ROPE || g.head_dim == 64) &&
                     (g.epi != EPI_GEGLU || g.N % 64 == 0);
   if (g.epi == EPI_ROPE && !mfma)
-    require(gBN % g.head_dim == 0, "gemm: ROPE epilogue needs head_dim dividing 64");
+    require(64 % g.head_dim == 0, "gemm: ROPE epilogue needs head_dim dividing 64");
   // split-K only for the residual epilogue: its few output tiles (N = D)
   // leave most CUs idle otherwise; the wider products (QKV, GEGLU) have
   // enough tiles, and a second epilogue kernel costs more than it saves
@@ -2262,11 +2113,8 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     check_launch("gemm_bf16_mfma");
     return;
   }
-  if (g.in_dtype == DT_BF16)
-    launch_generic<bf16_t>(g, st);
-  else
-    launch_generic<float>(g, st);
-  check_launch("gemm_generic");
+  launch_gemm_f32(g, st);
+  check_launch("gemm_f32");
 }
 
 }  // namespace sjh

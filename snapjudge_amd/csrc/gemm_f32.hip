@@ -1,0 +1,386 @@
+// gemm_f32.hip -- fp32-product GEMM for gfx950: out[M, N] = epi(A[M, K] . W[N, K]^T).
+//
+// Serves the fp32 numerics mode, the decision tail (scorer and act head, fp32
+// in every mode), LoRA, and the bf16 shapes that the bf16 kernels' tiling does
+// not cover (they are widened exactly on load).  Products and sums are fp32
+// throughout: v_mfma_f32_16x16x4_f32.
+//
+// What bounds it.  The fp32 matrix rate is a sixteenth of the bf16 one (a
+// 16x16x4 block takes 32 cycles), so operand bandwidth is not the limit once
+// the loads are coalesced.
+//  - gemm_f32_staged_kernel: 64x64 or 32x64 tiles, four waves, 32-deep K steps
+//    moved by direct-to-LDS loads (eight lanes take 128 contiguous bytes of a
+//    row) through a three-stage ring.
+//  - gemm_f32_split_kernel, for products too small to give every CU such a
+//    tile: 16x64 or 16x16 tiles whose eight waves each take an eighth of K and
+//    add their sums through LDS in wave order, so that the weights stream
+//    through as many CUs as there are and a wave's few steps are all in flight
+//    at once.  Operands go straight to registers in the MFMA's own layout; 16
+//    neighbouring lanes then read 16 different rows, which the vector cache
+//    serves at a quarter of its rate or less (64x64 tiles loaded this way ran
+//    the 1536 x 768 x 768 scorer in 51 us), so it is used only where latency,
+//    not that rate, is the limit.
+// Measured against the 64x64x16 FMA tiles both replace: the scorer's product of
+// one request, 16 x 768 x 768, 83 (mean of the tail's four products) -> 7.4 us;
+// of 96 questions, 1536 x 768 x 768, 85 (mean) -> 30 us (60 TFLOP/s; 8192 x
+// 3072 x 768 reaches 107 of the 154 that a large fp32 product of the vendor
+// library does); QKV of 569 rows 112 -> 32 us, the residual products 107 -> 21.
+// Both take the k values of a 16-deep group in the lanes' own order: lane
+// (r, q) holds row r's values 4 q + [0, 4) and MFMA j of the group takes the
+// lanes' j-th values, the same k on both sides.  The epilogue runs on the fp32
+// tile in LDS.
+#include <algorithm>
+#include <type_traits>
+
+#include "sjh_common.hpp"
+#include "sjh_host.hpp"
+#include "sjh_kernels.hpp"
+
+namespace sjh {
+
+namespace {
+
+// ---- epilogue over an fp32 BMxBN tile staged in LDS (row stride ldcs) ----
+template <int BM, int BN, int NT, typename OutT>
+__device__ __forceinline__ void tile_epilogue(const float* Cs, int ldcs, int m0, int tile_n,
+                                              const GemmArgs g) {
+  const int tid = threadIdx.x;
+  if (g.epi == EPI_GEGLU) {
+    constexpr int HB = BN / 2;
+    const int j0 = tile_n * HB;
+    OutT* out = static_cast<OutT*>(g.out);
+    for (int idx = tid; idx < BM * HB; idx += NT) {
+      const int r = idx / HB, c = idx - r * HB;
+      const int m = m0 + r, j = j0 + c;
+      if (m < g.M && j < g.N) {
+        const float in = Cs[r * ldcs + c], gate = Cs[r * ldcs + HB + c];
+        store_f32(out + static_cast<int64_t>(m) * g.ldo + j, gelu_out<OutT>(in) * gate);
+      }
+    }
+    return;
+  }
+  const int n0 = tile_n * BN;
+  for (int idx = tid; idx < BM * BN; idx += NT) {
+    const int r = idx / BN, c = idx - r * BN;
+    const int m = m0 + r, n = n0 + c;
+    if (m >= g.M || n >= g.N) continue;
+    float v = Cs[r * ldcs + c];
+    if (g.epi == EPI_RESID) {
+      if (g.bias) v += g.bias[n];
+      g.X[static_cast<int64_t>(m) * g.ldx + n] += v;
+      continue;
+    }
+    if (g.epi == EPI_ROPE) {
+      if (n < 2 * g.rope_dim) {
+        const int hd = g.head_dim, half = hd >> 1;
+        const int dd = n % hd;
+        const int64_t p = min(max(g.pos[m], 0), g.rope_rows - 1);
+        if (dd < half) {
+          const float x1 = Cs[r * ldcs + c + half];
+          const float cs = g.rope_cos[p * half + dd], sn = g.rope_sin[p * half + dd];
+          v = rope_lo(v, x1, cs, sn);
+        } else {
+          const int d2 = dd - half;
+          const float x0 = Cs[r * ldcs + c - half];
+          const float cs = g.rope_cos[p * half + d2], sn = g.rope_sin[p * half + d2];
+          v = rope_hi(x0, v, cs, sn);
+        }
+        if (n < g.rope_dim) v *= g.q_scale;
+      }
+    } else {
+      if (g.bias) v += g.bias[n];
+      if (g.act == 1)
+        v = gelu_out<OutT>(v);
+      else if (g.act == 2)
+        v = fmaxf(v, 0.f);
+    }
+    store_f32(static_cast<OutT*>(g.out) + static_cast<int64_t>(m) * g.ldo + n, v);
+  }
+}
+
+// W row feeding tile row i of column tile tile_n (GEGLU: first half of the
+// tile = input rows, second half = gate rows of the reference's [2F, K] Wi).
+template <int BN>
+__device__ __forceinline__ int64_t w_row(const GemmArgs g, int tile_n, int i) {
+  if (g.epi == EPI_GEGLU) {
+    constexpr int HB = BN / 2;
+    const int j = tile_n * HB + (i < HB ? i : i - HB);
+    const int jc = j < g.N ? j : g.N - 1;
+    return i < HB ? jc : static_cast<int64_t>(g.N) + jc;
+  }
+  const int n = tile_n * BN + i;
+  return n < g.N ? n : g.N - 1;
+}
+
+// Four k values of one operand row as fp32 (16- or 8-byte load).
+__device__ __forceinline__ f32x4_t load4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
+__device__ __forceinline__ f32x4_t load4(const bf16_t* p) {
+  const u32x2_t v = *reinterpret_cast<const u32x2_t*>(p);
+  return f32x4_t{__uint_as_float(v[0] << 16), __uint_as_float(v[0] & 0xffff0000u), __uint_as_float(v[1] << 16),
+                 __uint_as_float(v[1] & 0xffff0000u)};
+}
+template <typename T>
+__device__ __forceinline__ f32x4_t load4_upto(const T* p, int n) {
+  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (j < n) v[j] = load_f32(p + j);
+  return v;
+}
+
+// Tile of workgroup blockIdx.x.  XCDs get contiguous runs of tiles (workgroups
+// go round-robin over the 8 XCDs); the operand with fewer rows is the one that
+// every XCD reads whole.
+template <int BM, int BN>
+__device__ __forceinline__ void pick_tile(const GemmArgs& g, int launch_m, int& tile_m, int& tile_n) {
+  const int tiles_n = g.epi == EPI_GEGLU ? (g.N + BN / 2 - 1) / (BN / 2) : (g.N + BN - 1) / BN;
+  const int tiles_m = (launch_m + BM - 1) / BM;
+  const int nb = static_cast<int>(gridDim.x), bid = static_cast<int>(blockIdx.x);
+  const int xcd = bid & 7, per = nb >> 3, rem = nb & 7;
+  const int tile = xcd * per + min(xcd, rem) + (bid >> 3);
+  if (launch_m < g.N) {
+    tile_n = tile / tiles_m;
+    tile_m = tile - tile_n * tiles_m;
+  } else {
+    tile_m = tile / tiles_n;
+    tile_n = tile - tile_m * tiles_n;
+  }
+}
+
+// 16 x 16 TJ tiles, K cut into WGK slices of whole 16-deep steps, one wave
+// each, PD steps of operands in flight per wave.  vec_steps: leading steps that
+// may use vector loads (aligned rows).
+template <typename InT, typename OutT, int TJ, int WGK, int PD>
+__global__ __launch_bounds__(64 * WGK) void gemm_f32_split_kernel(GemmArgs g0, int vec_steps) {
+  GemmArgs g = g0;
+  if (g.M_dev) g.M = *g.M_dev;
+  constexpr int BM = 16, BN = 16 * TJ, NT = 64 * WGK, LDC = BN + 4;
+  __shared__ float Cs[WGK * BM * LDC];
+  int tile_m, tile_n;
+  pick_tile<BM, BN>(g, g0.M, tile_m, tile_n);
+  const int m0 = tile_m * BM;
+  if (m0 >= g.M) return;  // a row tile past the device row count (uniform)
+
+  const int tid = threadIdx.x, lane = tid & 63, wk = tid >> 6;
+  const int r16 = lane & 15, q4 = (lane >> 4) * 4;
+  const InT* ap = static_cast<const InT*>(g.A) + static_cast<int64_t>(min(m0 + r16, g.M - 1)) * g.lda + q4;
+  const InT* wp[TJ];
+#pragma unroll
+  for (int j = 0; j < TJ; ++j)
+    wp[j] = static_cast<const InT*>(g.W) + w_row<BN>(g, tile_n, j * 16 + r16) * g.ldw + q4;
+
+  f32x4_t acc[TJ];
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t a[PD], w[PD][TJ];
+  auto mac = [&](int u) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][c], w[u][j][c], acc[j], 0, 0, 0);
+  };
+  auto load = [&](int s, int u) {
+    a[u] = load4(ap + 16 * s);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) w[u][j] = load4(wp[j] + 16 * s);
+  };
+
+  // steps [s0, s1) of this wave: vector loads up to vec_steps, then guarded
+  // scalar loads (unaligned rows, and the step that K ends in)
+  const int steps = (g.K + 15) >> 4, chunk = (steps + WGK - 1) / WGK;
+  const int s0 = wk * chunk, s1 = min(s0 + chunk, steps);
+  const int n = min(s1, vec_steps) - s0;
+  int i = 0;
+#pragma unroll
+  for (int u = 0; u < PD; ++u)
+    if (u < n) load(s0 + u, u);
+  for (; i + 2 * PD <= n; i += PD)
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {
+      mac(u);
+      load(s0 + i + u + PD, u);
+    }
+#pragma unroll
+  for (int u = 0; u < PD; ++u)
+    if (i + u < n) {
+      mac(u);
+      if (i + u + PD < n) load(s0 + i + u + PD, u);
+    }
+#pragma unroll
+  for (int u = 0; u < PD; ++u)
+    if (i + PD + u < n) mac(u);
+  for (int s = max(s0, vec_steps); s < s1; ++s) {
+    const int left = g.K - 16 * s - q4;  // k values of this lane's four that exist
+    a[0] = load4_upto(ap + 16 * s, left);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) w[0][j] = load4_upto(wp[j] + 16 * s, left);
+    mac(0);
+  }
+
+  // accumulator lane (r, q): column r, rows 4 q + [0, 4) of a block
+  float* C = Cs + wk * BM * LDC;
+#pragma unroll
+  for (int j = 0; j < TJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) C[(q4 + e) * LDC + j * 16 + r16] = acc[j][e];
+  __syncthreads();
+  for (int idx = tid; idx < BM * BN; idx += NT) {  // the slices' sums, in order
+    const int o = (idx / BN) * LDC + idx % BN;
+    float v = Cs[o];
+#pragma unroll
+    for (int k = 1; k < WGK; ++k) v += Cs[k * BM * LDC + o];
+    Cs[o] = v;
+  }
+  __syncthreads();
+  tile_epilogue<BM, BN, NT, OutT>(Cs, LDC, m0, tile_n, g);
+}
+
+// BM x 64 tiles of fp32 operands, four waves in 2 x 2.  vec: 16-byte aligned
+// rows; otherwise, and for the last partial K step, rows are staged value by
+// value.
+template <typename OutT, int BM>
+__global__ __launch_bounds__(256) void gemm_f32_staged_kernel(GemmArgs g0, int vec) {
+  GemmArgs g = g0;
+  if (g.M_dev) g.M = *g.M_dev;
+  constexpr int BN = 64, BK = 32, NS = 3, RB = BK * 4, ROWS = BM + BN, LDC = BN + 4;
+  constexpr int TI = BM / 32, TJ = 2, G = ROWS / 32;  // load instructions (8 rows each) per wave and stage
+  constexpr int STAGE = ROWS * RB;
+  static_assert(NS * STAGE >= BM * LDC * 4, "the epilogue's tile reuses the ring");
+  __shared__ __attribute__((aligned(16))) char ring[NS * STAGE];
+  int tile_m, tile_n;
+  pick_tile<BM, BN>(g, g0.M, tile_m, tile_n);
+  const int m0 = tile_m * BM;
+  if (m0 >= g.M) return;  // a row tile past the device row count (uniform)
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, q = lane >> 4;
+  const float* A = static_cast<const float*>(g.A);
+  const float* W = static_cast<const float*>(g.W);
+  auto row_ptr = [&](int r) {
+    return r < BM ? A + static_cast<int64_t>(min(m0 + r, g.M - 1)) * g.lda : W + w_row<BN>(g, tile_n, r - BM) * g.ldw;
+  };
+  // 16-byte chunk c of row r sits at slot c ^ swz(r): 16 consecutive rows at one
+  // chunk then fall into 16 different 16-byte bank groups
+  auto swz = [](int r) { return (r >> 1) & 7; };
+  const float* src[G];
+#pragma unroll
+  for (int i = 0; i < G; ++i) {
+    const int r = 8 * (wave + 4 * i) + (lane >> 3);
+    src[i] = row_ptr(r) + 4 * ((lane & 7) ^ swz(r));
+  }
+  auto issue = [&](int kt, int slot) {
+#pragma unroll
+    for (int i = 0; i < G; ++i) load_lds16(src[i] + kt * BK, ring + slot * STAGE + (wave + 4 * i) * 1024);
+  };
+
+  f32x4_t acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int key = swz(r16);  // (a block's first row is a multiple of 16)
+  const char* a_row = ring + (wm * TI * 16 + r16) * RB;
+  const char* w_rowp = ring + (BM + wn * TJ * 16 + r16) * RB;
+  auto compute = [&](int slot) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int off = slot * STAGE + ((4 * h + q) ^ key) * 16;
+      f32x4_t a[TI], w[TJ];
+#pragma unroll
+      for (int i = 0; i < TI; ++i) a[i] = *reinterpret_cast<const f32x4_t*>(a_row + i * 16 * RB + off);
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) w[j] = *reinterpret_cast<const f32x4_t*>(w_rowp + j * 16 * RB + off);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][c], w[j][c], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  const int nk = vec ? g.K / BK : 0;
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (s < nk) issue(s, s);
+  int slot = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    if (kt + 1 < nk)
+      wait_vmcnt<G*(NS - 2)>();
+    else
+      wait_vmcnt<0>();
+    wait_lgkm0();  // this wave's reads of the slot that is refilled next
+    __builtin_amdgcn_s_barrier();
+    if (kt + NS - 1 < nk) issue(kt + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+    compute(slot);
+    slot = slot + 1 == NS ? 0 : slot + 1;
+  }
+  for (int k0 = nk * BK; k0 < g.K; k0 += BK) {
+    __syncthreads();
+    for (int idx = tid; idx < ROWS * 8; idx += 256) {
+      const int r = idx >> 3, c = idx & 7;
+      const f32x4_t v = load4_upto(row_ptr(r) + k0 + 4 * c, g.K - k0 - 4 * c);
+      *reinterpret_cast<f32x4_t*>(ring + r * RB + (c ^ swz(r)) * 16) = v;
+    }
+    __syncthreads();
+    compute(0);
+  }
+  __syncthreads();
+  float* Cs = reinterpret_cast<float*>(ring);
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        Cs[((wm * TI + i) * 16 + 4 * q + e) * LDC + (wn * TJ + j) * 16 + r16] = acc[i][j][e];
+  __syncthreads();
+  tile_epilogue<BM, BN, 256, OutT>(Cs, LDC, m0, tile_n, g);
+}
+
+unsigned tiles_of(const GemmArgs& g, int BM, int BN) {
+  const int64_t tiles_n = g.epi == EPI_GEGLU ? (g.N + BN / 2 - 1) / (BN / 2) : (g.N + BN - 1) / BN;
+  const int64_t tiles = tiles_n * ((g.M + BM - 1) / BM);
+  require(tiles < (int64_t{1} << 31), "gemm: too many tiles");
+  return static_cast<unsigned>(tiles);
+}
+
+template <typename InT, typename OutT>
+void launch_typed(const GemmArgs& g, hipStream_t st) {
+  const uintptr_t align = 4 * sizeof(InT) - 1;
+  const bool vec = g.lda % 4 == 0 && g.ldw % 4 == 0 && (reinterpret_cast<uintptr_t>(g.A) & align) == 0 &&
+                   (reinterpret_cast<uintptr_t>(g.W) & align) == 0;
+  // Staged tiles once there are enough for three CUs in four (N = 768, 575
+  // rows: 21 us a product against 28 split); 64 rows each where there are
+  // several rounds of them anyway (fewer operand bytes per product), 32 below,
+  // so that the last round is shorter.
+  const unsigned t32 = tiles_of(g, 32, 64);
+  if (std::is_same<InT, float>::value && t32 >= 192) {
+    if (t32 >= 2048)
+      gemm_f32_staged_kernel<OutT, 64><<<tiles_of(g, 64, 64), 256, 0, st>>>(g, vec);
+    else
+      gemm_f32_staged_kernel<OutT, 32><<<t32, 256, 0, st>>>(g, vec);
+    return;
+  }
+  // 16x16 tiles where 16x64 ones would leave CUs idle and the epilogue (bias,
+  // activation, residual) needs no pairs of columns
+  const int vec_steps = vec ? g.K / 16 : 0;
+  if (tiles_of(g, 16, 64) < 256 && (g.epi == EPI_STORE || g.epi == EPI_RESID))
+    gemm_f32_split_kernel<InT, OutT, 1, 8, 6><<<tiles_of(g, 16, 16), 512, 0, st>>>(g, vec_steps);
+  else
+    gemm_f32_split_kernel<InT, OutT, 4, 8, 6><<<tiles_of(g, 16, 64), 512, 0, st>>>(g, vec_steps);
+}
+
+}  // namespace
+
+void launch_gemm_f32(const GemmArgs& g, hipStream_t st) {
+  const bool bf_out = g.out_dtype == DT_BF16;
+  if (g.in_dtype == DT_BF16)
+    bf_out ? launch_typed<bf16_t, bf16_t>(g, st) : launch_typed<bf16_t, float>(g, st);
+  else
+    bf_out ? launch_typed<float, bf16_t>(g, st) : launch_typed<float, float>(g, st);
+}
+
+}  // namespace sjh

@@ -112,6 +112,9 @@ constexpr int kLnBlock = 256;
 constexpr bool kLnFoldEnabled = false;
 constexpr int kLnMaxBlocks = 4;  // D <= 1024 (c1 rows hold 8 bf16, blocks past 4 zero)
 void launch_gemm(const GemmArgs& g, hipStream_t st);
+// launch_gemm's fp32-product path (checked arguments): any shape and
+// alignment, fp32 or bf16 operands, every epilogue (RoPE: head_dim divides 64).
+void launch_gemm_f32(const GemmArgs& g, hipStream_t st);
 // Whether a GEMM of these arguments takes the persistent kernel, the only
 // one that can produce or consume a folded LayerNorm.
 bool gemm_takes_ln_fold(const GemmArgs& g);
