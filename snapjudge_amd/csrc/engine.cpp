@@ -704,6 +704,7 @@ void Engine::ensure_workspace(int Tb, int Bb) {
   ws_.seq = seqinfo_.as<int32_t>();
   ws_.tok_pos = tok_pos_.as<int>();
   ws_.tok_seq = tok_seq_.as<int>();
+  ws_.X = X_.as<float>();
   ws_.Y = Y_.get();
   ws_.QKV = QKV_.get();
   ws_.O = O_.get();
@@ -829,17 +830,28 @@ std::vector<std::tuple<const char*, double, int64_t>> Engine::profile_totals() {
   return v;
 }
 
-void Engine::gemm(const char* name, const GemmArgs& g0, const Ws& w, hipStream_t st) {
+namespace {
+// Launches g on the short-batch kernels where they take it.
+bool try_gemm_short(const GemmArgs& g0, hipStream_t st) {
+  GemmArgs g = g0;
+  g.M_dev = nullptr;
+  if (!gemm_short_ok(g)) return false;
+  launch_gemm_short(g, st);
+  return true;
+}
+}  // namespace
+
+void Engine::gemm(const char* name, const GemmArgs& g0, const Ws& w, hipStream_t st, bool short_rows) {
   GemmArgs g = g0;
   g.partial = w.partial;
   g.partial_cap = w.partial_cap;
   prof_begin(st);
-  launch_gemm(g, st);
+  if (!short_rows || !try_gemm_short(g, st)) launch_gemm(g, st);
   prof_end(name, st);
 }
 
 void Engine::resid_gemm_ln(const char* gname, const GemmArgs& g0, const char* lname, LnArgs a,
-                           const Ws& w, hipStream_t st) {
+                           const Ws& w, hipStream_t st, bool short_rows) {
   GemmArgs g = g0;
   g.partial = w.partial;
   g.partial_cap = w.partial_cap;
@@ -852,8 +864,9 @@ void Engine::resid_gemm_ln(const char* gname, const GemmArgs& g0, const char* ln
   folded.xio = g.X;
   folded.n_parts = 1;
   prof_begin(st);
-  const int S = g.M <= 256 && ln_takes_parts(folded) ? launch_gemm_resid_partials(g, st) : 0;
-  if (S == 0) launch_gemm(g, st);
+  const bool done = short_rows && try_gemm_short(g, st);
+  const int S = !done && g.M <= 256 && ln_takes_parts(folded) ? launch_gemm_resid_partials(g, st) : 0;
+  if (!done && S == 0) launch_gemm(g, st);
   prof_end(gname, st);
   if (S > 0) {  // X is updated by the layer norm: X += sum of the splits (+ bias)
     folded.n_parts = S;
@@ -931,6 +944,12 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
                        D % kAttnWoCols == 0 && D <= 1024 && w.partial &&
                        static_cast<int64_t>(H_) * T * D <= w.partial_cap;
 
+  // a short batch's residual stream stays in the workspace (all Tb rows); the
+  // final norm writes the caller's rows
+  const bool shortb = w.X && short_batch(T);
+  float* const out = X;
+  if (shortb) X = w.X;
+
   // src/model.cpp:332-340: X = LN(emb[ids]); layer 0 reads X itself.  BERT
   // family (src/sj_model.cpp:220-237): X = LN(word[ids] + pos[position] ; w, b)
   const bool bert = arch_ == ARCH_BERT;
@@ -983,7 +1002,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
     a.y_dtype = adt;
     a.ld_y = D;
     a.M = T;
-    a.M_dev = T_dev;
+    a.M_dev = shortb ? nullptr : T_dev;  // (all rows exist: nothing waits for the row count)
     a.D = D;
     return a;
   };
@@ -995,7 +1014,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
   final_args.w = final_norm_.as<float>();
   final_args.b = final_norm_b_.as<float>();
   final_args.eps = eps_;
-  final_args.x_out = X;
+  final_args.x_out = out;
   final_args.ld_x = D;
   final_args.M = T;
   final_args.M_dev = T_dev;
@@ -1051,7 +1070,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
       if (bert) {
         g.epi = EPI_STORE;
         g.bias = ly.wqkv_b.as<float>();
-        gemm("gemm_qkv_bias", g, w, st);
+        gemm("gemm_qkv_bias", g, w, st, shortb);
       } else {
         g.epi = EPI_ROPE;
         g.pos = w.tok_pos;
@@ -1067,7 +1086,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
           g.ln_c2 = ly.ln1_c2.as<float>();
           g.ln_eps = eps_;
         }
-        gemm("gemm_qkv_rope", g, w, st);
+        gemm("gemm_qkv_rope", g, w, st, shortb);
       }
     }
     {  // attention (src/model.cpp:381)
@@ -1137,7 +1156,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
       a.y_dtype = adt;
       a.ld_y = D;
       a.M = T;
-      a.M_dev = T_dev;
+      a.M_dev = shortb ? nullptr : T_dev;
       a.D = D;
       if (attn_wo) {  // attention wrote the heads' partials of O . Wo^T
         LnArgs f = a;
@@ -1157,7 +1176,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
       } else if (rln_resid(g, a, w)) {
         gemm("gemm_wo_resid_ln", g, w, st);
       } else {
-        resid_gemm_ln("gemm_wo_resid", g, "mlp_norm", a, w, st);
+        resid_gemm_ln("gemm_wo_resid", g, "mlp_norm", a, w, st, shortb);
       }
     }
     {  // G = geglu(Y . Wi^T) (src/model.cpp:394); BERT: G = gelu(Y . W1^T + b1)
@@ -1180,7 +1199,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
         g.epi = EPI_STORE;
         g.bias = ly.wi_b.as<float>();
         g.act = 1;
-        gemm("gemm_w1_gelu", g, w, st);
+        gemm("gemm_w1_gelu", g, w, st, shortb);
       } else {
         g.epi = EPI_GEGLU;
         if (fold) {
@@ -1189,7 +1208,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
           g.ln_c2 = ly.ln2_c2.as<float>();
           g.ln_eps = eps_;
         }
-        gemm("gemm_wi_geglu", g, w, st);
+        gemm("gemm_wi_geglu", g, w, st, shortb);
       }
     }
     {  // X += G . Wo2^T (src/model.cpp:395-397)
@@ -1220,12 +1239,13 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
         if (rln_resid(g, a, w))
           gemm("gemm_wo2_resid_ln", g, w, st);
         else
-          resid_gemm_ln("gemm_wo2_resid", g, "attn_norm", a, w, st);
+          resid_gemm_ln("gemm_wo2_resid", g, "attn_norm", a, w, st, shortb);
       } else {
-        resid_gemm_ln("gemm_wo2_resid", g, "final_norm", final_args, w, st);
+        resid_gemm_ln("gemm_wo2_resid", g, "final_norm", final_args, w, st, shortb);
       }
     }
   }
+  X = out;
   if (lora_r_ > 0) {  // h += (h . A^T) . B^T (src/model.cpp:402-407)
     GemmArgs g;
     g.A = X;
@@ -1271,6 +1291,7 @@ void Engine::enqueue_head_layers(const BatchPlan& p, const Ws& w, float* X, hipS
   launch_add_row_embedding(X, D, type_emb_.as<float>(), seq_start + 3 * Bb, w.tok_seq, T, T_dev,
                            D, st);
   const float scale = 1.0f / std::sqrt(static_cast<float>(Dh_));
+  const bool shortb = short_batch(T);  // (X is a workspace buffer of Tb rows)
   for (const HeadDev& hd : head_) {
     LnArgs a;
     a.in = X;
@@ -1283,7 +1304,7 @@ void Engine::enqueue_head_layers(const BatchPlan& p, const Ws& w, float* X, hipS
     a.y_dtype = adt;
     a.ld_y = D;
     a.M = T;
-    a.M_dev = T_dev;
+    a.M_dev = shortb ? nullptr : T_dev;
     a.D = D;
     ln("head_norm1", a, st);
 
@@ -1302,7 +1323,7 @@ void Engine::enqueue_head_layers(const BatchPlan& p, const Ws& w, float* X, hipS
     g.ldo = 3 * D;
     g.out_dtype = adt;
     g.bias = hd.in_b.as<float>();
-    gemm("head_in_proj", g, w, st);
+    gemm("head_in_proj", g, w, st, shortb);
 
     AttnArgs at;
     at.q = w.QKV;
@@ -1339,7 +1360,7 @@ void Engine::enqueue_head_layers(const BatchPlan& p, const Ws& w, float* X, hipS
     go.X = X;
     go.ldx = D;
     go.bias = hd.out_b.as<float>();
-    gemm("head_out_proj", go, w, st);
+    gemm("head_out_proj", go, w, st, shortb);
 
     LnArgs a2 = a;
     a2.w = hd.n2w.as<float>();
@@ -1362,7 +1383,7 @@ void Engine::enqueue_head_layers(const BatchPlan& p, const Ws& w, float* X, hipS
     g1.out_dtype = adt;
     g1.bias = hd.l1b.as<float>();
     g1.act = head_act_;
-    gemm("head_linear1", g1, w, st);
+    gemm("head_linear1", g1, w, st, shortb);
 
     GemmArgs g2;
     g2.A = w.G;
@@ -1378,7 +1399,7 @@ void Engine::enqueue_head_layers(const BatchPlan& p, const Ws& w, float* X, hipS
     g2.X = X;
     g2.ldx = D;
     g2.bias = hd.l2b.as<float>();
-    gemm("head_linear2", g2, w, st);
+    gemm("head_linear2", g2, w, st, shortb);
   }
 }
 
@@ -1534,6 +1555,8 @@ size_t Engine::scratch_layout(const BatchPlan& p, Ws& ws) const {
   };
   const size_t seq = take(seq_table_ints(p.Bb) * 4);
   const size_t tok_pos = take(t * 4), tok_seq = take(t * 4);
+  const bool shortb = short_batch(p.Tb);
+  const size_t X = take(shortb ? t * D * 4 : 0);
   const size_t Y = take(t * D * as), QKV = take(t * 3 * D * as), O = take(t * D * as);
   const size_t G = take(t * static_cast<size_t>(F_) * as);
   const size_t Z = lora_r_ > 0 ? take(t * static_cast<size_t>(lora_r_) * 4) : 0;
@@ -1546,6 +1569,7 @@ size_t Engine::scratch_layout(const BatchPlan& p, Ws& ws) const {
   ws.seq = reinterpret_cast<int32_t*>(scratch_ + seq);
   ws.tok_pos = reinterpret_cast<int*>(scratch_ + tok_pos);
   ws.tok_seq = reinterpret_cast<int*>(scratch_ + tok_seq);
+  ws.X = shortb ? reinterpret_cast<float*>(scratch_ + X) : nullptr;
   ws.Y = scratch_ + Y;
   ws.QKV = scratch_ + QKV;
   ws.O = scratch_ + O;

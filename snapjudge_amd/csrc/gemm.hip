@@ -1961,6 +1961,20 @@ void launch_splitk_epi(const GemmArgs& g, dim3 grid, hipStream_t st) {
   kern<<<grid, 256, lds, st>>>(g);
 }
 
+}  // namespace
+
+void split_k_slices(int M, int N, int K, int& slices, int& chunk) {
+  const int tiles = ((M + kSkBM - 1) / kSkBM) * ((N + kSkBN - 1) / kSkBN);
+  const int nk = K / kBK;
+  // enough workgroups to cover the CUs, at least two K steps per split
+  slices = std::min(std::max(1, (512 + tiles - 1) / tiles), std::max(1, nk / 2));
+  slices = std::min(slices, 16);
+  chunk = (nk + slices - 1) / slices;
+  slices = (nk + chunk - 1) / chunk;
+}
+
+namespace {
+
 // Launches the split-K product (partials only) and returns the number of
 // splits, or 0 (nothing launched) when the workspace is too small or K too
 // short to split.
@@ -1970,12 +1984,8 @@ int launch_splitk_partials(GemmArgs& g, hipStream_t st) {
   if (g.epi == EPI_GEGLU && g.N % (kSkBN / 2) != 0) return 0;
   const int tiles_n = g.epi == EPI_GEGLU ? g.N / (kSkBN / 2) : (g.N + kSkBN - 1) / kSkBN;
   const int tiles = ((g.M + kSkBM - 1) / kSkBM) * tiles_n;
-  const int nk = g.K / kBK;
-  // enough workgroups to cover the CUs, at least two K steps per split
-  int S = std::min(std::max(1, (512 + tiles - 1) / tiles), std::max(1, nk / 2));
-  S = std::min(S, 16);
-  g.k_chunk = (nk + S - 1) / S;
-  S = (nk + g.k_chunk - 1) / g.k_chunk;
+  int S = 0;
+  split_k_slices(g.M, g.n_w, g.K, S, g.k_chunk);
   if (S < 2 || static_cast<int64_t>(S) * g.M * g.n_w > g.partial_cap) return 0;
   dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(S));
   switch (g.epi) {

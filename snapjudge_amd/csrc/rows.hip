@@ -16,10 +16,7 @@ namespace sjh {
 namespace {
 
 constexpr int kLnWaves = 4;        // rows per workgroup
-#ifndef SJH_LN_PARTS_WAVES
-#define SJH_LN_PARTS_WAVES 1
-#endif
-constexpr int kLnPartsWaves = SJH_LN_PARTS_WAVES;  // rows per workgroup of the split-K sums
+constexpr int kLnSpreadRows = 512;  // up to this many rows: one per workgroup
 constexpr int kLnMaxPerLane = 64;  // D <= 4096 (64 lanes x 64 values)
 
 // LayerNorm as src/tensor.cpp:54-79: mean and population variance
@@ -373,12 +370,8 @@ __global__ __launch_bounds__(64 * WPB) void ln_vec_kernel(LnArgs a) {
   }
 }
 
-template <int NV, typename InT, typename ResT>
-void ln_vec_dispatch_out(const LnArgs& a, hipStream_t st) {
-  // Rows (waves) per workgroup.  The split-K partial sums run on short
-  // batches only (M <= 256): each row there streams its partial rows, so
-  // the rows are spread over kLnPartsWaves-wave workgroups.
-  constexpr int WPB = std::is_same<ResT, PartsRes>::value ? kLnPartsWaves : kLnWaves;
+template <int NV, typename InT, typename ResT, int WPB>
+void ln_vec_launch(const LnArgs& a, hipStream_t st) {
   dim3 grid((a.M + WPB - 1) / WPB), block(64 * WPB);
   const bool full = a.D == 256 * NV;
   if (a.y_dtype == DT_BF16)
@@ -387,6 +380,17 @@ void ln_vec_dispatch_out(const LnArgs& a, hipStream_t st) {
   else
     full ? ln_vec_kernel<NV, true, InT, ResT, float, WPB><<<grid, block, 0, st>>>(a)
          : ln_vec_kernel<NV, false, InT, ResT, float, WPB><<<grid, block, 0, st>>>(a);
+}
+
+template <int NV, typename InT, typename ResT>
+void ln_vec_dispatch_out(const LnArgs& a, hipStream_t st) {
+  // Rows (waves) per workgroup: one while that still leaves CUs without a row
+  // (and for split-K partial sums, whose rows stream many partial rows), four
+  // for longer batches
+  if (std::is_same<ResT, PartsRes>::value || a.M <= kLnSpreadRows)
+    ln_vec_launch<NV, InT, ResT, 1>(a, st);
+  else
+    ln_vec_launch<NV, InT, ResT, kLnWaves>(a, st);
 }
 
 template <typename InT, typename ResT>

@@ -112,6 +112,17 @@ constexpr int kLnBlock = 256;
 constexpr bool kLnFoldEnabled = false;
 constexpr int kLnMaxBlocks = 4;  // D <= 1024 (c1 rows hold 8 bf16, blocks past 4 zero)
 void launch_gemm(const GemmArgs& g, hipStream_t st);
+// The short-batch kernels (gemm_short.hip): QKV + RoPE, Wi + GEGLU and plain
+// products (bias, activation; K a multiple of 256 up to 1024, bf16 output) and
+// residual products (K a multiple of 64), bf16 rows and bf16 or fp8 weights, a
+// multiple of 32 rows up to kShortMaxRows.  All M rows of the launch are read
+// and written (no M_dev): the buffers hold them.
+constexpr int kShortMaxRows = 256;
+// The K slices of a residual product of a short batch: slices of chunk 64-deep
+// units each (the last may be shorter).
+void split_k_slices(int M, int N, int K, int& slices, int& chunk);
+bool gemm_short_ok(const GemmArgs& g);
+void launch_gemm_short(const GemmArgs& g, hipStream_t st);
 // launch_gemm's fp32-product path (checked arguments): any shape and
 // alignment, fp32 or bf16 operands, every epilogue (RoPE: head_dim divides 64).
 void launch_gemm_f32(const GemmArgs& g, hipStream_t st);
