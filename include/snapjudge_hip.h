@@ -182,7 +182,7 @@ int sjh_model_forward_shared(sjh_model* m, const int64_t* ids, const int64_t* ma
 /* Encoder on a batch already resident in device memory: d_ids [T] int32 holds
  * the B sequences back to back, h_lens [B] (host) their lengths, T = sum.
  * Writes the final hidden states [T, D] fp32 to d_hidden.  Work is enqueued on
- * `stream` (NULL: the model's own stream); the call does not synchronize. */
+ * `stream` (NULL: the legacy null stream); the call does not synchronize. */
 int sjh_model_encode_device(sjh_model* m, const int32_t* d_ids, const int32_t* h_lens, int32_t B,
                             float* d_hidden, sjh_stream_t stream);
 

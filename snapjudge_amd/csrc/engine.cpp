@@ -275,14 +275,12 @@ Engine::Engine(const ModelSource& src, const sjh_options& o) {
   hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
   hip_check(hipEventCreateWithFlags(&ev_done_, hipEventDisableTiming), "hipEventCreate");
   hip_check(hipEventCreateWithFlags(&ev_upload_, hipEventDisableTiming), "hipEventCreate");
-  hip_check(hipEventCreateWithFlags(&ev_null_, hipEventDisableTiming), "hipEventCreate");
   try {
     scratch_ = scratch_for_device(dev_);
     stage_weights(src);
     hip_check(hipStreamSynchronize(stream_), "weight staging");
   } catch (...) {  // the destructor does not run for a constructor that throws
     (void)hipStreamSynchronize(stream_);
-    (void)hipEventDestroy(ev_null_);
     (void)hipEventDestroy(ev_done_);
     (void)hipEventDestroy(ev_upload_);
     (void)hipStreamDestroy(stream_);
@@ -302,8 +300,7 @@ Engine::~Engine() {
     (void)hipEventDestroy(p.b);
   }
   for (hipEvent_t e : ev_pool_) (void)hipEventDestroy(e);
-  if (done_recorded_) (void)hipEventSynchronize(ev_done_);
-  if (ev_null_) (void)hipEventDestroy(ev_null_);
+  if (last_done_ == ev_done_ && ev_done_) (void)hipEventSynchronize(ev_done_);  // (else a graph's, above)
   if (ev_done_) (void)hipEventDestroy(ev_done_);
   if (ev_upload_) (void)hipEventDestroy(ev_upload_);
   if (stream_) (void)hipStreamDestroy(stream_);
@@ -665,7 +662,7 @@ BatchPlan Engine::plan_lens(const int32_t* h_lens, int B) const {
 void Engine::ensure_workspace(int Tb, int Bb) {
   if (Tb <= cap_T_ && Bb <= cap_B_) return;
   // every earlier call's work (on any stream) has finished with the old buffers
-  if (done_recorded_) hip_check(hipEventSynchronize(ev_done_), "sync before workspace growth");
+  if (last_done_) hip_check(hipEventSynchronize(last_done_), "sync before workspace growth");
   const int nT = std::max(Tb, cap_T_ + cap_T_ / 4);
   const int nB = std::max(Bb, cap_B_);
   const size_t t = static_cast<size_t>(std::max(nT, 1));
@@ -755,12 +752,12 @@ void Engine::set_seq_table(const BatchPlan& p, const int32_t* h_lens, int32_t* t
 }
 
 void Engine::begin_call(hipStream_t st) {
-  if (done_recorded_) hip_check(hipStreamWaitEvent(st, ev_done_, 0), "order after the previous call");
+  if (last_done_) hip_check(hipStreamWaitEvent(st, last_done_, 0), "order after the previous call");
 }
 
 void Engine::end_call(hipStream_t st) {
   hip_check(hipEventRecord(ev_done_, st), "record call end");
-  done_recorded_ = true;
+  last_done_ = ev_done_;
 }
 
 // ------------------------------------------------------------------ launches --
@@ -1409,11 +1406,11 @@ void Engine::run_device(const BatchPlan& p, const Ws& w, const int32_t* d_ids, f
   if (head) enqueue_head_layers(p, w, X, st);
 }
 
-void Engine::run_device_maybe_graph(const BatchPlan& p, const int32_t* d_ids, float* X,
+bool Engine::run_device_maybe_graph(const BatchPlan& p, const int32_t* d_ids, float* X,
                                     bool head, hipStream_t st) {
   if (!use_graphs_ || profile_) {
     run_device(p, ws_, d_ids, X, head, st);
-    return;
+    return false;
   }
   // one graph per bucket and buffer set: the batch's own sizes and lengths
   // reach the kernels through the sequence table, written before the launch
@@ -1437,16 +1434,18 @@ void Engine::run_device_maybe_graph(const BatchPlan& p, const int32_t* d_ids, fl
       drop_graph(lru->second);
       graphs_.erase(lru);
     }
+    // (the null stream cannot be captured; a graph launches on any stream)
+    hipStream_t cs = st ? st : stream_;
     hipGraph_t graph = nullptr;
-    hip_check(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "begin capture");
+    hip_check(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal), "begin capture");
     try {
-      run_device(p, ws_, d_ids, X, head, st);
+      run_device(p, ws_, d_ids, X, head, cs);
     } catch (...) {
-      (void)hipStreamEndCapture(st, &graph);
+      (void)hipStreamEndCapture(cs, &graph);
       if (graph) (void)hipGraphDestroy(graph);
       throw;
     }
-    hip_check(hipStreamEndCapture(st, &graph), "end capture");
+    hip_check(hipStreamEndCapture(cs, &graph), "end capture");
     Graph g;
     hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
@@ -1464,10 +1463,13 @@ void Engine::run_device_maybe_graph(const BatchPlan& p, const int32_t* d_ids, fl
   it->second.last_use = ++graph_clock_;
   hip_check(hipGraphLaunch(it->second.exec, st), "graph launch");
   hip_check(hipEventRecord(it->second.done, st), "record graph launch");
+  last_done_ = it->second.done;
+  return true;
 }
 
 void Engine::drop_graph(Graph& g) {
   if (g.exec) (void)hipGraphExecDestroy(g.exec);
+  if (g.done && g.done == last_done_) last_done_ = nullptr;  // (its launch has ended)
   if (g.done) (void)hipEventDestroy(g.done);
   g.exec = nullptr;
   g.done = nullptr;
@@ -1522,24 +1524,16 @@ void Engine::encode_device(const int32_t* d_ids, const int32_t* h_lens, int B, f
   hip_check(hipSetDevice(dev_), "hipSetDevice");
   if (B <= 0) return;
   require(d_ids && h_lens && d_hidden, "encode_device: null argument");
-  // NULL selects the model's own stream, ordered after and before the legacy
-  // null stream so that NULL behaves like the default stream for the caller.
-  hipStream_t st = stream ? stream : stream_;
+  // NULL is the legacy null stream itself (the work was once sent through the
+  // model's own stream, with an event wait on either side: ~45 us a call)
   BatchPlan p = plan_lens(h_lens, B);
   if (p.T == 0) return;
   ensure_workspace(p.Tb, p.Bb);
-  begin_call(st);
-  if (!stream) {
-    hip_check(hipEventRecord(ev_null_, nullptr), "record null stream");
-    hip_check(hipStreamWaitEvent(st, ev_null_, 0), "wait null stream");
-  }
-  set_seq_table(p, h_lens, ws_.seq, st);
-  run_device_maybe_graph(p, d_ids, d_hidden, false, st);
-  end_call(st);
-  if (!stream) {
-    hip_check(hipEventRecord(ev_null_, st), "record model stream");
-    hip_check(hipStreamWaitEvent(nullptr, ev_null_, 0), "null stream waits");
-  }
+  begin_call(stream);
+  set_seq_table(p, h_lens, ws_.seq, stream);
+  // (a graph's own event marks the end of its launch: a second one would cost
+  // another ~5 us between calls)
+  if (!run_device_maybe_graph(p, d_ids, d_hidden, false, stream)) end_call(stream);
 }
 
 size_t Engine::scratch_layout(const BatchPlan& p, Ws& ws) const {
@@ -1602,26 +1596,17 @@ void Engine::encode_device_noalloc(const int32_t* d_ids, const int32_t* h_lens, 
          " bytes of scratch; the fixed scratch array holds " + std::to_string(kScratchBytes) +
          " bytes, about " + std::to_string(kScratchBytes / per_tok) + " tokens of this model");
   }
-  hipStream_t st = stream ? stream : stream_;
-  begin_call(st);
-  if (!stream) {
-    hip_check(hipEventRecord(ev_null_, nullptr), "record null stream");
-    hip_check(hipStreamWaitEvent(st, ev_null_, 0), "wait null stream");
-  }
+  begin_call(stream);
   quiet_ = true;
   try {
-    launch_seq_table(h_lens, p.B, p.Bb, w.seq, st);
-    run_device(p, w, d_ids, d_hidden, false, st);
+    launch_seq_table(h_lens, p.B, p.Bb, w.seq, stream);
+    run_device(p, w, d_ids, d_hidden, false, stream);
   } catch (...) {
     quiet_ = false;
     throw;
   }
   quiet_ = false;
-  end_call(st);
-  if (!stream) {
-    hip_check(hipEventRecord(ev_null_, st), "record model stream");
-    hip_check(hipStreamWaitEvent(nullptr, ev_null_, 0), "null stream waits");
-  }
+  end_call(stream);
 }
 
 void Engine::forward(const int64_t* ids, const int64_t* mask, const int64_t* marker_pos,

@@ -190,7 +190,8 @@ class Engine {
   // `head`, through the decision-head layers)
   void run_device(const BatchPlan& p, const Ws& w, const int32_t* d_ids, float* X, bool head,
                   hipStream_t st);
-  void run_device_maybe_graph(const BatchPlan& p, const int32_t* d_ids, float* X, bool head,
+  // (true: the work ran as a graph, whose event marks its end)
+  bool run_device_maybe_graph(const BatchPlan& p, const int32_t* d_ids, float* X, bool head,
                               hipStream_t st);
   void enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_ids, float* X,
                        hipStream_t st);
@@ -285,12 +286,12 @@ class Engine {
   uint64_t ws_gen_ = 0;
 
   hipStream_t stream_ = nullptr;
-  hipEvent_t ev_null_ = nullptr;  // orders NULL-stream callers of encode_device
-  // ev_done_: the end of the last call's device work, on whichever stream it
-  // ran; every call waits for it first.  ev_upload_: the last copy out of
-  // the pinned staging buffer, awaited before the buffer is rewritten.
-  hipEvent_t ev_done_ = nullptr, ev_upload_ = nullptr;
-  bool done_recorded_ = false, upload_recorded_ = false;
+  // last_done_: the event at the end of the last call's device work, on
+  // whichever stream it ran (ev_done_, or the event of the graph it launched);
+  // every call waits for it first.  ev_upload_: the last copy out of the pinned
+  // staging buffer, awaited before the buffer is rewritten.
+  hipEvent_t last_done_ = nullptr, ev_done_ = nullptr, ev_upload_ = nullptr;
+  bool upload_recorded_ = false;
   std::map<std::vector<int64_t>, Graph> graphs_;
   uint64_t graph_clock_ = 0;
   int64_t n_captures_ = 0, n_replays_ = 0;
