@@ -879,7 +879,7 @@ bool Engine::rln_resid(GemmArgs& g, const LnArgs& a, const Ws& w) const {
       a.in_dtype != DT_F32 || a.y_dtype != DT_BF16 || !a.y_out || a.x_out || a.xio || a.resid || a.ids ||
       a.add || a.M != g.M || a.D != g.N)
     return false;
-  if (!gemm_takes_rln(g)) return false;
+  if (!gemm_takes_rln(g, rln_spin_ == 1)) return false;  // (the one-poll mode: wherever it can run)
   g.rln_y = a.y_out;
   g.rln_ldy = a.ld_y;
   g.rln_w = a.w;

@@ -122,19 +122,35 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
   } else if constexpr (EPI == EPI_GEGLU) {
     OutT* out = static_cast<OutT*>(g.out);
     const int c0 = tile_n * (BN / 2) + wn * (WN / 2) + l32;
+    // the values of eight rows, then their stores: a bounds check before each
+    // value would make the GELUs wait for one another
+    const bool full = m0 + (wm + 1) * WM <= g.M && c0 - l32 + WN / 2 <= g.N;  // uniform
+    auto body = [&](auto checked) {
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = row_base + i * 32 + 8 * (e >> 2) + (e & 3);
-        if (m >= g.M) continue;
-        OutT* orow = out + static_cast<int64_t>(m) * g.ldo;
+        for (int e0 = 0; e0 < 16; e0 += 8) {
+          float v[8][TJ / 2];
 #pragma unroll
-        for (int j = 0; j < TJ / 2; ++j) {
-          const int col = c0 + j * 32;
-          if (col < g.N) store_f32(orow + col, gelu_out<OutT>(acc[i][j][e]) * acc[i][j + TJ / 2][e]);
+          for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int j = 0; j < TJ / 2; ++j) v[e][j] = gelu_out<OutT>(acc[i][j][e0 + e]) * acc[i][j + TJ / 2][e0 + e];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int m = row_base + i * 32 + 8 * ((e0 + e) >> 2) + ((e0 + e) & 3);
+            OutT* orow = out + static_cast<int64_t>(m) * g.ldo;
+#pragma unroll
+            for (int j = 0; j < TJ / 2; ++j) {
+              const int col = c0 + j * 32;
+              if (!decltype(checked)::value || (m < g.M && col < g.N)) store_f32(orow + col, v[e][j]);
+            }
+          }
         }
-      }
+    };
+    if (full)
+      body(std::false_type{});
+    else
+      body(std::true_type{});
   } else if constexpr (EPI == EPI_RESID) {
     // X += acc (+ bias).  The X reads of a group of RG rows are all issued
     // before the first add, so a group costs one memory round trip rather
@@ -165,9 +181,23 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
           for (int e = 0; e < RG; ++e) {
             const int r = i * 32 + 8 * ((e0 + e) >> 2) + ((e0 + e) & 3);
             const char* xr = xw + static_cast<uint32_t>(r * ld4 + lo);
+            // a partial tile reads its last row and column again rather than
+            // branch per element (a branch would wait for each load)
+            const float* xc = nullptr;
+            if constexpr (decltype(checked)::value) xc = g.X + static_cast<int64_t>(min(rw + r + 4 * hb, g.M - 1)) * g.ldx;
 #pragma unroll
-            for (int j = 0; j < TJ; ++j)
-              xv[e][j] = in(r, j) ? *reinterpret_cast<const float*>(xr + j * 128) : 0.f;
+            for (int j = 0; j < TJ; ++j) {
+              if constexpr (decltype(checked)::value)
+                xv[e][j] = xc[min(c0 + j * 32 + l32, g.N - 1)];
+              else
+                xv[e][j] = *reinterpret_cast<const float*>(xr + j * 128);
+            }
+          }
+          if constexpr (decltype(checked)::value) {
+#pragma unroll
+            for (int e = 0; e < RG; ++e)
+#pragma unroll
+              for (int j = 0; j < TJ; ++j) consume(xv[e][j]);
           }
 #pragma unroll
           for (int e = 0; e < RG; ++e) {
@@ -328,19 +358,26 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
 #pragma unroll
       for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int r = i * 32 + 8 * (e >> 2) + (e & 3);
-          if (decltype(checked)::value && rw + r + 4 * hb >= g.M) continue;
-          char* orow = const_cast<char*>(ow) + static_cast<uint32_t>(r * ldb + lo);
+        for (int e0 = 0; e0 < 16; e0 += 8) {
+          float v[8][TJ];  // eight rows' values, then their stores (see GEGLU)
 #pragma unroll
-          for (int j = 0; j < TJ; ++j) {
-            if (decltype(checked)::value && c0 + j * 32 + l32 >= g.N) continue;
-            float v = acc[i][j][e] + bv[j];
-            if constexpr (ACT == 1)
-              v = gelu_out<OutT>(v);
-            else if constexpr (ACT == 2)
-              v = fmaxf(v, 0.f);
-            store_f32(reinterpret_cast<OutT*>(orow + j * 32 * EB), v);
+          for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+              v[e][j] = acc[i][j][e0 + e] + bv[j];
+              if constexpr (ACT == 1)
+                v[e][j] = gelu_out<OutT>(v[e][j]);
+              else if constexpr (ACT == 2)
+                v[e][j] = fmaxf(v[e][j], 0.f);
+            }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int r = i * 32 + 8 * ((e0 + e) >> 2) + ((e0 + e) & 3);
+            char* orow = const_cast<char*>(ow) + static_cast<uint32_t>(r * ldb + lo);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+              if (!decltype(checked)::value || (rw + r + 4 * hb < g.M && c0 + j * 32 + l32 < g.N))
+                store_f32(reinterpret_cast<OutT*>(orow + j * 32 * EB), v[e][j]);
           }
         }
     };
@@ -880,7 +917,7 @@ __device__ __forceinline__ void resid_rln_epilogue(const GemmArgs& g, f32x16_t (
 // stages form a ring; the loads for stage kt + NS - 1 are issued right after
 // the barrier that opens iteration kt, so NS - 1 stages are in flight while
 // stage kt is consumed.
-template <int BM, int BN, int WGM, int WGN, int NS, int BK>
+template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8 = false>
 struct DTile {
   static constexpr int NW = WGM * WGN;
   static constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -888,10 +925,12 @@ struct DTile {
   static constexpr int RB = BK * 2;                // bytes per tile row
   static constexpr int CPR = BK / 8;               // 16-byte chunks per row
   static constexpr int RPI = 1024 / RB;            // rows per load instruction
-  static constexpr int GROUPS = (BM + BN) / RPI;   // load instructions per stage
+  static constexpr int WRB = W8 ? BK : RB;         // bytes per W row
+  static constexpr int GROUPS = BM / RPI + BN * WRB / 1024;  // load instructions per stage
   static constexpr int G = GROUPS / NW;            // ... per wave
-  static constexpr int STAGE_BYTES = (BM + BN) * RB;
+  static constexpr int STAGE_BYTES = BM * RB + BN * WRB;
   static_assert(BK == 32 || BK == 64, "K step is 32 or 64");
+  static_assert(!W8 || BK == 64, "fp8 rows: 64-byte steps");
   static_assert(G * NW == GROUPS && BM % RPI == 0, "row groups must split evenly over waves");
   static_assert(TI >= 1 && TJ >= 1, "tile too small");
   static_assert(NS >= 2 && NS * STAGE_BYTES <= 160 * 1024, "LDS ring does not fit");
@@ -909,9 +948,9 @@ template <typename OutT>
 __device__ void splitk_output(const GemmArgs& g, int S, int m, int n);
 
 template <int BM, int BN, int WGM, int WGN, int NS, int BK, int EPI, typename OutT,
-          bool SPLITK = false>
+          bool SPLITK = false, bool W8 = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_dma_kernel(GemmArgs g0) {
-  using TT = DTile<BM, BN, WGM, WGN, NS, BK>;
+  using TT = DTile<BM, BN, WGM, WGN, NS, BK, W8>;
   const GemmArgs g = resolve_rows(g0);
   constexpr int TI = TT::TI, TJ = TT::TJ, G = TT::G, RB = TT::RB, CPR = TT::CPR;
   constexpr int KS = BK / 16;  // MFMA K steps per stage
@@ -932,22 +971,32 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_dma_kernel(GemmArgs 
   // this wave's row groups: q = wave + NW * i; lane moves tile row
   // RPI * q + lane / CPR into chunk slot lane % CPR, reading the logical
   // chunk that the swizzle maps there
-  const bf16_t* src[G];
+  // (fp8 W rows: 16 rows of 64 bytes per instruction, four lanes each)
+  const char* src[G];
+  bool w8_src[G];  // uniform: a source that advances BK bytes per step, not 2 BK
   const int lrow = lane / CPR, cslot = lane % CPR;
 #pragma unroll
   for (int i = 0; i < G; ++i) {
-    const int r = TT::RPI * (wave + TT::NW * i) + lrow;
+    const int q = __builtin_amdgcn_readfirstlane(wave) + TT::NW * i;
+    w8_src[i] = W8 && q >= BM / TT::RPI;
+    if (w8_src[i]) {
+      const int r = (q - BM / TT::RPI) * 16 + (lane >> 2);
+      src[i] = static_cast<const char*>(g.W) + mfma_w_row<BN, TT::WN, EPI>(g, tile_n, r) * g.ldw +
+               ((lane & 3) ^ ((r >> 2) & 3)) * 16;
+      continue;
+    }
+    const int r = TT::RPI * q + lrow;
     const int gchunk = cslot ^ TT::swz(r);
     if (r < BM)
-      src[i] = A + static_cast<int64_t>(min(m0 + r, g.M - 1)) * g.lda + gchunk * 8;
+      src[i] = reinterpret_cast<const char*>(A + static_cast<int64_t>(min(m0 + r, g.M - 1)) * g.lda + gchunk * 8);
     else
-      src[i] = W + mfma_w_row<BN, TT::WN, EPI>(g, tile_n, r - BM) * g.ldw + gchunk * 8;
+      src[i] = reinterpret_cast<const char*>(W + mfma_w_row<BN, TT::WN, EPI>(g, tile_n, r - BM) * g.ldw + gchunk * 8);
   }
   auto issue = [&](int kt, int buf) {
     char* base = dsmem + buf * TT::STAGE_BYTES;
 #pragma unroll
     for (int i = 0; i < G; ++i)
-      load_lds16(static_cast<const void*>(src[i] + kt * BK), base + (wave + TT::NW * i) * 1024);
+      load_lds16(src[i] + (w8_src[i] ? kt * BK : kt * BK * 2), base + (wave + TT::NW * i) * 1024);
   };
 
   f32x16_t acc[TI][TJ];
@@ -971,7 +1020,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_dma_kernel(GemmArgs 
   // operand rows of this lane; tile bases are multiples of 32, so the
   // swizzle key of row base + l32 is that of l32
   const int xr = TT::swz(l32);
-  const int a_row0 = (wm * TT::WM + l32) * RB, w_row0 = (BM + wn * TT::WN + l32) * RB;
+  const int a_row0 = (wm * TT::WM + l32) * RB, w_row0 = BM * RB + (wn * TT::WN + l32) * TT::WRB;
   for (int kt = 0; kt < nk; ++kt) {
     if (kt + NS - 2 < nk)
       wait_vmcnt<G * (NS - 2)>();
@@ -983,14 +1032,26 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_dma_kernel(GemmArgs 
     // operand fragments double-buffered across the K steps so the LDS reads
     // of step s + 1 are in flight during the MFMAs of step s
     bf16x8_t af[2][TI], bw[2][TJ];
+    u32x4_t wraw[2][TJ];  // fp8 codes of a step pair, by pair parity
     auto frag = [&](int s, int buf) {
-      const int coff = ((2 * s + hb) ^ xr) * 16;
+      // fp8: a lane's 16-byte read of W holds its codes of two steps, so the
+      // chunks of a pair go 0, 2 | 1, 3 (as in the persistent kernel)
+      const int coff = ((W8 ? 4 * (s >> 1) + 2 * hb + (s & 1) : 2 * s + hb) ^ xr) * 16;
 #pragma unroll
       for (int i = 0; i < TI; ++i)
         af[buf][i] = *reinterpret_cast<const bf16x8_t*>(sb + a_row0 + i * 32 * RB + coff);
 #pragma unroll
-      for (int j = 0; j < TJ; ++j)
-        bw[buf][j] = *reinterpret_cast<const bf16x8_t*>(sb + w_row0 + j * 32 * RB + coff);
+      for (int j = 0; j < TJ; ++j) {
+        if constexpr (W8) {
+          u32x4_t& r = wraw[(s >> 1) & 1][j];
+          if ((s & 1) == 0)
+            r = *reinterpret_cast<const u32x4_t*>(sb + w_row0 + j * 32 * TT::WRB +
+                                                  (((s & 2) + hb) ^ ((l32 >> 2) & 3)) * 16);
+          bw[buf][j] = (s & 1) ? fp8x8_to_bf16(r[2], r[3]) : fp8x8_to_bf16(r[0], r[1]);
+        } else {
+          bw[buf][j] = *reinterpret_cast<const bf16x8_t*>(sb + w_row0 + j * 32 * RB + coff);
+        }
+      }
     };
     frag(0, 0);
 #pragma unroll
@@ -1022,6 +1083,16 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_dma_kernel(GemmArgs 
     }
   }
 
+  if constexpr (W8) {  // row n of W stands for code * w_scale[n]
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      const float sc = g.w_scale[mfma_w_row<BN, TT::WN, EPI>(g, tile_n, wn * TT::WN + j * 32 + l32)];
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] *= sc;
+    }
+  }
   if constexpr (!SPLITK) {
     gemm_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT>(g, acc, m0, tile_n, wm, wn, l32, hb);
   } else {
@@ -1714,6 +1785,12 @@ int num_cus() {
   return n;
 }
 
+// Output tiles of BM rows by BN rows of W.
+int64_t count_tiles(const GemmArgs& g, int BM, int BN) {
+  const int n = g.epi == EPI_GEGLU ? BN / 2 : BN;
+  return ((int64_t{g.N} + n - 1) / n) * ((int64_t{g.M} + BM - 1) / BM);
+}
+
 template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8, int EPI, typename OutT, int LNF>
 void launch_pers_kernel(const GemmArgs& g, hipStream_t st) {
   // (+ 1 KB of row positions for the RoPE epilogue, + a folded LayerNorm's
@@ -1780,10 +1857,10 @@ void launch_pers(const GemmArgs& g, hipStream_t st) {
   }
 }
 
-template <int BM, int BN, int WGM, int WGN, int NS, int BK, int EPI, typename OutT>
+template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8, int EPI, typename OutT>
 void launch_mfma_kernel(const GemmArgs& g, dim3 grid, hipStream_t st) {
-  constexpr int lds = NS * DTile<BM, BN, WGM, WGN, NS, BK>::STAGE_BYTES;
-  auto kern = gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, BK, EPI, OutT>;
+  constexpr int lds = NS * DTile<BM, BN, WGM, WGN, NS, BK, W8>::STAGE_BYTES;
+  auto kern = gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, BK, EPI, OutT, false, W8>;
   static bool attr_set = false;  // per instantiation; the attribute is per function
   if (!attr_set) {
     hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1794,41 +1871,29 @@ void launch_mfma_kernel(const GemmArgs& g, dim3 grid, hipStream_t st) {
   kern<<<grid, 64 * WGM * WGN, lds, st>>>(g);
 }
 
-template <int BM, int BN, int WGM, int WGN, int NS, int BK, int EPI>
+template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8, int EPI>
 void launch_mfma_tile(const GemmArgs& g, hipStream_t st) {
-  const int tiles_n = EPI == EPI_GEGLU ? g.N / (BN / 2) : (g.N + BN - 1) / BN;
-  const int64_t tiles = static_cast<int64_t>(tiles_n) * ((g.M + BM - 1) / BM);
+  const int64_t tiles = count_tiles(g, BM, BN);
   require(tiles < (int64_t{1} << 31), "gemm: too many tiles");
   dim3 grid(static_cast<unsigned>(tiles));
   if (g.out_dtype == DT_BF16 || EPI == EPI_RESID)
-    launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, EPI, bf16_t>(g, grid, st);
+    launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI, bf16_t>(g, grid, st);
   else
-    launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, EPI, float>(g, grid, st);
+    launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI, float>(g, grid, st);
 }
 
-template <int BM, int BN, int WGM, int WGN, int NS, int BK>
+template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8>
 void launch_mfma_epi(const GemmArgs& g, hipStream_t st) {
   switch (g.epi) {
-    case EPI_STORE: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, EPI_STORE>(g, st); break;
-    case EPI_RESID: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, EPI_RESID>(g, st); break;
-    case EPI_ROPE: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, EPI_ROPE>(g, st); break;
-    default: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, EPI_GEGLU>(g, st); break;
+    case EPI_STORE: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, W8, EPI_STORE>(g, st); break;
+    case EPI_RESID: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, W8, EPI_RESID>(g, st); break;
+    case EPI_ROPE: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, W8, EPI_ROPE>(g, st); break;
+    default: launch_mfma_tile<BM, BN, WGM, WGN, NS, BK, W8, EPI_GEGLU>(g, st); break;
   }
 }
 
-#ifndef SJH_GEMM_BIG
-#define SJH_GEMM_BIG 256, 256, 4, 4, 2, 64
-#endif
-#ifndef SJH_GEMM_MID
-#define SJH_GEMM_MID 128, 128, 2, 2, 2, 64
-#endif
-
-// Tile shapes by row count (BM, BN, wave grid, ring stages, K step): 256x256
-// with 16 waves of 64x64 (4 waves per SIMD hide the LDS and MFMA latencies)
-// for the throughput shapes; 128x128 with 4 waves for mid-size batches;
-// 64x64 with 2 waves of 32x64 and a 4-stage ring for short ones (batch-1
-// latency): more workgroups spread the weight reads over the CUs, and three
-// stages in flight cover the load latency that bounds such a short loop.
+// Tile shapes (BM, BN, wave grid, ring stages, K step).  Every shape gives the
+// same bits; pick_tile() chooses by how many tiles each cuts a product into.
 #ifndef SJH_GEMM_PERS
 #define SJH_GEMM_PERS 256, 256, 4, 4, 2, 64
 #endif
@@ -1840,11 +1905,8 @@ void launch_mfma_epi(const GemmArgs& g, hipStream_t st) {
 #define SJH_GEMM_PERS_FP8 256, 256, 4, 4, 3, 64
 #endif
 
-#ifndef SJH_GEMM_SMALL
-#define SJH_GEMM_SMALL 64, 64, 2, 1, 4, 64
-#endif
-// Up to SJH_SMALL32_MAX_M rows (batch-1 latency), the GEGLU and plain
-// products take 32-column tiles: a CU streams W at ~25 GB/s at most, so half
+// Up to SJH_SMALL32_MAX_M rows, the GEGLU, plain and head_dim-64 RoPE products
+// that gemm_short.hip does not take have 32-column tiles: a CU streams W at ~25 GB/s at most, so half
 // the W rows per workgroup on twice the workgroups shortens the K loop
 // (batch-1 Wi + GEGLU 10.2 -> 8.1 us per launch).  A GEGLU tile's input and
 // gate rows meet in the epilogue by a lane swap, and so do the rotation
@@ -1872,21 +1934,67 @@ bool pers_ok(const GemmArgs& g) {
          (g.epi != EPI_ROPE || static_cast<int64_t>(g.rope_rows) * 128 < (int64_t{1} << 32));
 }
 
+// What bounds these products between the latency of a few rows and the matrix
+// pipes of a full chip is each CU's intake: ~50 GB/s from L2 into LDS however
+// many stages are in flight, so a product wants its tiles on every CU, then
+// tiles as large as that leaves (fewer bytes per output).  Per launch, us, M x
+// N x K, on the shapes' neighbours (bench of every shape at 320 to 18 432 rows):
+//  T64     64x64, 2 waves, 4 stages, up to a tile per CU: 1024 x 768 x 1152 9.9
+//          (128x64 10.7, 128x128 12.3)
+//  T128x64 4 waves, 3 stages, up to a tile per CU: 2304 x 768 x 1152 11.3
+//          (128x128 13.2), 640 x 2304 x 768 9.2 (64x64 10.1)
+//  T128D   128x128, 8 waves of 32x64, 4 stages (one workgroup per CU), up to a
+//          tile per CU: 2304 x 1024 x 2624 26.5 (2 stages 31.6), 4032 x 768 x
+//          1152 15.2 (16.9)
+//  T128    the same with 2 stages, two workgroups per CU, for more tiles: 3072 x
+//          2304 x 768 RoPE 19.1 (4 waves of 64x64 19.7), 6120 x 768 x 768
+//          residual 18.0 (the persistent kernel's 72 tiles 28.5); plain and GEGLU
+//          products keep four waves of 64x64 (1501 x 3072 x 768 GELU 18.1, eight
+//          waves 18.6)
+//  TPERS   the persistent 256x256 kernel from kPersMinTiles tiles on: 3072 x 2624
+//          GEGLU x 1024 (246 tiles) 35.0 (T128 40.6), 18 432 x 2304 x 768 72.8
+//          (88); 3072 x 3072 x 1024 (144 tiles) 30.8 against 29.8
+enum Tile { T64, T128x64, T128D, T128, TPERS };
+constexpr int kPersMinTiles = 160;
+// a residual product that also finishes the LayerNorm saves its launch: 12 000 x
+// 768 x (768 / 1152) (141 tiles) 42.5 us with it, 43.5 on T128 and two launches
+constexpr int kRlnMinTiles = 128;
+
+Tile pick_tile(const GemmArgs& g) {
+  if (g.rln_y || g.ln_y || g.ln_stats_in) return TPERS;  // (checked by launch_gemm)
+  const int cus = num_cus();
+  if (count_tiles(g, 64, 64) <= cus) return T64;
+  if (count_tiles(g, 128, 64) <= cus) return T128x64;
+  if (count_tiles(g, 256, 256) >= kPersMinTiles && pers_ok(g)) return TPERS;
+  return count_tiles(g, 128, 128) <= cus ? T128D : T128;
+}
+
+template <bool W8>
 void launch_mfma(const GemmArgs& g, hipStream_t st) {
-  if (g.M >= 4096 && pers_ok(g))
-    launch_pers<SJH_GEMM_PERS, false>(g, st);
-  else if (g.M >= 4096 && (g.epi != EPI_GEGLU || g.N % 128 == 0))
-    launch_mfma_epi<SJH_GEMM_BIG>(g, st);
-  else if (g.M >= 1024)
-    launch_mfma_epi<SJH_GEMM_MID>(g, st);
-  else if (g.M <= SJH_SMALL32_MAX_M && g.epi == EPI_GEGLU)
-    launch_mfma_tile<SJH_GEMM_SMALL32, EPI_GEGLU>(g, st);
-  else if (g.M <= SJH_SMALL32_MAX_M && g.epi == EPI_STORE)
-    launch_mfma_tile<SJH_GEMM_SMALL32, EPI_STORE>(g, st);
-  else if (g.M <= SJH_SMALL32_MAX_M && g.epi == EPI_ROPE && g.head_dim == 64 && g.N % 64 == 0)
-    launch_mfma_tile<SJH_GEMM_SMALL32, EPI_ROPE>(g, st);
-  else
-    launch_mfma_epi<SJH_GEMM_SMALL>(g, st);
+  if (!W8 && g.M <= SJH_SMALL32_MAX_M) {
+    if (g.epi == EPI_GEGLU) return launch_mfma_tile<SJH_GEMM_SMALL32, false, EPI_GEGLU>(g, st);
+    if (g.epi == EPI_STORE) return launch_mfma_tile<SJH_GEMM_SMALL32, false, EPI_STORE>(g, st);
+    if (g.epi == EPI_ROPE && g.head_dim == 64 && g.N % 64 == 0)
+      return launch_mfma_tile<SJH_GEMM_SMALL32, false, EPI_ROPE>(g, st);
+  }
+  switch (pick_tile(g)) {
+    case T64: launch_mfma_epi<64, 64, 2, 1, 4, 64, W8>(g, st); break;
+    case T128x64: launch_mfma_epi<128, 64, 4, 1, 3, 64, W8>(g, st); break;
+    case T128D: launch_mfma_epi<128, 128, 4, 2, 4, 64, W8>(g, st); break;
+    case T128:  // eight waves where the epilogue also reads (residual rows, RoPE tables)
+      switch (g.epi) {
+        case EPI_STORE: launch_mfma_tile<128, 128, 2, 2, 2, 64, W8, EPI_STORE>(g, st); break;
+        case EPI_GEGLU: launch_mfma_tile<128, 128, 2, 2, 2, 64, W8, EPI_GEGLU>(g, st); break;
+        case EPI_RESID: launch_mfma_tile<128, 128, 4, 2, 2, 64, W8, EPI_RESID>(g, st); break;
+        default: launch_mfma_tile<128, 128, 4, 2, 2, 64, W8, EPI_ROPE>(g, st); break;
+      }
+      break;
+    default:
+      if constexpr (W8)
+        launch_pers<SJH_GEMM_PERS_FP8, true>(g, st);
+      else
+        launch_pers<SJH_GEMM_PERS, false>(g, st);
+  }
 }
 
 // ------------------------------------------------------------------ split-K
@@ -2029,17 +2137,18 @@ bool gemm_takes_ln_fold(const GemmArgs& g) {
     return g.in_dtype == DT_BF16 && g.w_scale && aligned16(g.w_scale) && g.K % 64 == 0 &&
            g.lda % 8 == 0 && g.ldw % 16 == 0 && aligned16(g.A) && aligned16(g.W) && pers_ok(g) &&
            (g.epi != EPI_ROPE || g.head_dim == 64);
-  return g.w_dtype == DT_BF16 && mfma_ok(g) && g.M >= 4096 && pers_ok(g);  // launch_mfma's first choice
+  return g.w_dtype == DT_BF16 && mfma_ok(g) && g.M >= 4096 && pers_ok(g);
 }
 
-bool gemm_takes_rln(const GemmArgs& g) {
+bool gemm_takes_rln(const GemmArgs& g, bool any_tiles) {
   if (g.epi != EPI_RESID || g.w_dtype != DT_BF16 || g.M <= 0 || g.N % kLnBlock != 0 ||
       g.N / kLnBlock > kLnMaxBlocks || !g.A || !g.W || !g.X)
     return false;
-  if (!(mfma_ok(g) && g.M >= 4096 && pers_ok(g))) return false;  // launch_mfma's persistent path
+  if (!(mfma_ok(g) && g.M >= 4096 && pers_ok(g))) return false;
   // one round: every tile a workgroup of its own, all resident at once
   const int64_t tiles = static_cast<int64_t>(g.N / kLnBlock) * ((g.M + 255) / 256);
-  return tiles <= static_cast<int64_t>(pers_occupancy<SJH_GEMM_PERS, false>()) * num_cus();
+  return (any_tiles || tiles >= kRlnMinTiles) &&
+         tiles <= static_cast<int64_t>(pers_occupancy<SJH_GEMM_PERS, false>()) * num_cus();
 }
 
 int launch_gemm_resid_partials(const GemmArgs& g0, hipStream_t st) {
@@ -2077,7 +2186,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
       fail("gemm: unknown epilogue");
   }
   if (g.rln_y) {
-    require(gemm_takes_rln(g), "gemm: the residual epilogue finishes a LayerNorm only on one round of 256 x 256 "
+    require(gemm_takes_rln(g, true), "gemm: the residual epilogue finishes a LayerNorm only on one round of 256 x 256 "
                                "bf16 tiles with N a multiple of 256 up to 1024");
     require(g.rln_w && g.rln_mom && g.rln_sync && g.rln_ldy >= g.N && g.rln_spin > 0 && g.rln_eps > 0.f &&
                 !g.ln_y && !g.ln_stats_in,
@@ -2095,7 +2204,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
             "gemm: a folded LayerNorm's consumer needs K % 256 == 0, K <= 1024, c1 rows and moments");
   }
   if (g.w_dtype == DT_FP8) {
-    // fp8 weights: the persistent kernel only (16-byte fp8 rows chunks)
+    // fp8 weights: 16-byte chunks of the codes' rows
     require(g.in_dtype == DT_BF16, "gemm: fp8 weights need bf16 activations");
     require(g.w_scale && aligned16(g.w_scale), "gemm: fp8 weights need per-row scales");
     require(g.K % 64 == 0 && g.lda % 8 == 0 && g.ldw % 16 == 0 && aligned16(g.A) &&
@@ -2103,7 +2212,10 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
             "gemm: fp8 weights need K % 64 == 0 and 16-byte aligned rows");
     require(pers_ok(g), "gemm: fp8 weights need N % 4 == 0, 16-byte aligned outputs and operands under 4 GiB");
     require(g.epi != EPI_ROPE || g.head_dim == 64, "gemm: fp8 RoPE epilogue needs head_dim 64");
-    launch_pers<SJH_GEMM_PERS_FP8, true>(g, st);
+    if (g.epi == EPI_GEGLU && g.N % 64 != 0)
+      launch_pers<SJH_GEMM_PERS_FP8, true>(g, st);  // (the other tiles take whole GEGLU columns)
+    else
+      launch_mfma<true>(g, st);
     check_launch("gemm_fp8w");
     return;
   }
@@ -2119,7 +2231,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   // enough tiles, and a second epilogue kernel costs more than it saves
   if (mfma && g.partial && g.M <= SJH_SPLITK_MAX_M && g.epi == EPI_RESID && launch_splitk(g, st)) return;
   if (mfma) {
-    launch_mfma(g, st);
+    launch_mfma<false>(g, st);
     check_launch("gemm_bf16_mfma");
     return;
   }

@@ -146,6 +146,9 @@ __global__ __launch_bounds__(256) void gemm_short_kernel(GemmArgs g) {
   __builtin_amdgcn_sched_barrier(0);
 
   const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, q = lane >> 4;
+  // 8-value chunk of a 32-deep step that this lane's quarter takes: in order,
+  // or 0, 2, 1, 3 for fp8 weights (the persistent kernel's order)
+  const int qc = W8 ? (q == 1 ? 2 : q == 2 ? 1 : q) : q;
   f32x4_t acc[TI];
 #pragma unroll
   for (int t = 0; t < TI; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -166,15 +169,15 @@ __global__ __launch_bounds__(256) void gemm_short_kernel(GemmArgs g) {
       for (int h = 0; h < 2; ++h) {
         bf16x8_t w;
         if constexpr (W8) {
-          const int r = wn * 16 + r16, c = 4 * h + q;  // 8-byte piece c of the row's eight
+          const int r = wn * 16 + r16, c = 4 * h + qc;  // 8-byte piece c of the row's eight
           const u32x2_t v = *reinterpret_cast<const u32x2_t*>(sw + r * 64 + ((c >> 1) ^ ((r >> 2) & 3)) * 16 + (c & 1) * 8);
           w = fp8x8_to_bf16(v[0], v[1]);
         } else {
-          w = *reinterpret_cast<const bf16x8_t*>(sw + (wn * 16 + r16) * 128 + ((4 * h + q) ^ ((r16 >> 1) & 7)) * 16);
+          w = *reinterpret_cast<const bf16x8_t*>(sw + (wn * 16 + r16) * 128 + ((4 * h + qc) ^ ((r16 >> 1) & 7)) * 16);
         }
 #pragma unroll
         for (int t = 0; t < TI; ++t) {
-          const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(sa + t * 2048 + ((4 * h + q) ^ ((r16 >> 1) & 7)) * 16);
+          const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(sa + t * 2048 + ((4 * h + qc) ^ ((r16 >> 1) & 7)) * 16);
           acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w, acc[t], 0, 0, 0);
         }
       }

@@ -136,11 +136,12 @@ bool gemm_takes_ln_fold(const GemmArgs& g);
 void launch_ln_fold_consts(const void* W, int w_dtype, const float* w_scale, int n_w, int K,
                            const float* ln_w, const float* ln_b, uint16_t* c1, float* c2,
                            hipStream_t st);
-// Whether the residual epilogue can finish the next LayerNorm for these
+// Whether the residual epilogue finishes the next LayerNorm for these
 // arguments (GemmArgs::rln_y): the persistent bf16 kernel, N a multiple of 256
 // up to 1024, and at most one tile per workgroup, so that all of a panel's
-// tiles run at once.
-bool gemm_takes_rln(const GemmArgs& g);
+// tiles run at once; of those, the launches whose tiles occupy enough of the
+// chip for it to pay, or (any_tiles) all of them.
+bool gemm_takes_rln(const GemmArgs& g, bool any_tiles);
 // Short batches (M <= 256) of a residual GEMM (EPI_RESID, bf16 MFMA path):
 // launches only the split-K product into g.partial and returns the number of
 // splits S >= 2; the caller then adds the splits with the layer norm that
