@@ -17,13 +17,8 @@
 // straight from the row-major V tile through transposed LDS reads
 // (ds_read_b64_tr_b16).
 //
-// Generic path (fp32 or bf16, head_dim 8/16/32/64/128): one thread per query,
-// K/V tiles of 32 keys in LDS (broadcast reads), blocked online softmax with
-// expf.  It serves the fp32 parity mode.
-//
-// Masking follows src/tensor.cpp:186-192: query i sees keys
-// [0, k_len) (full) or [max(0, i-w), min(k_len, i+w+1)) (window w).  A query
-// with no visible key yields zeros, as the reference does for len = 0.
+// fp32, and bf16 of other head dims (8/16/32/128): attn_f32_kernel, fp32
+// products on the matrix cores.
 #include <type_traits>
 
 #include "sjh_common.hpp"
@@ -756,101 +751,162 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const int32_t* table, i
   }
 }
 
-// ------------------------------------------------------------------ generic
-constexpr int gQ = 128;   // queries per workgroup (one per thread)
-constexpr int gKey = 32;  // keys per LDS tile
+// ------------------------------------------------------------- fp32 products
+// Attention with fp32 products (the fp32 mode) and of head dims other than 64
+// (bf16 values widened exactly).  A workgroup takes 64 queries of one head, 16
+// per wave, over 64-key tiles of K and V in LDS (32 at head_dim 128), the next
+// tile's rows in flight in registers meanwhile.
+//
+// S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x4_f32: lane (c, q) of an
+// accumulator holds column c (a query) and rows 4 q + [0, 4) (keys, head dims).
+// So a query's softmax is within its lane but for one exchange over the four
+// lanes that share it, and P goes from S^T's accumulator straight into the
+// second product: its MFMA e takes keys 4 q + e, V's rows read in that order.
+// Bound by the fp32 matrix rate (a tile is 128 MFMAs of 32 cycles a wave).
+// Against one thread per query with scalar FMAs: 575 tokens in five rows, 12
+// heads of 64 (two thirds of the layers windowed), 156 -> 15.8 us a launch.
+constexpr int fQ = 64;  // queries per workgroup
 
 template <typename T, int DH>
-__global__ __launch_bounds__(gQ) void attn_generic_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a, int vec) {
+  constexpr int DP = DH < 16 ? 16 : DH;  // padded with zeros to one MFMA block
+  constexpr int KT = DP > 64 ? 32 : 64, NB = KT / 16, ND = DP / 16;
+  constexpr int LDR = DP + 4;  // rows 4 q + e of V, and 16 rows of K, on different banks
+  constexpr int NL = KT * DP / 4 / 256 > 0 ? KT * DP / 4 / 256 : 1;  // 4-value pieces per thread and operand
   const int b = a.seq_order ? a.seq_order[blockIdx.z] : static_cast<int>(blockIdx.z);
   const int h = blockIdx.y;
   const int qlen = a.q_len ? a.q_len[b] : a.uniform_L;
-  const int q0 = blockIdx.x * gQ;
+  const int q0 = blockIdx.x * fQ;
   if (q0 >= qlen) return;
   // keys never extend past the rows a sequence owns (a caller's k_len > L in
   // the padded layout is clamped rather than read out of bounds)
   const int klen = a.seq_start ? a.k_len[b] : max(0, min(a.k_len[b], a.uniform_L));
   const int64_t row0 = a.seq_start ? a.seq_start[b] : static_cast<int64_t>(b) * a.uniform_L;
-  const int tid = threadIdx.x;
-  const int qi = q0 + tid;
-  const bool active = qi < qlen;
-
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
+  const int qi = q0 + wave * 16 + c;
   const T* Q = static_cast<const T*>(a.q) + h * DH;
   const T* K = static_cast<const T*>(a.k) + h * DH;
   const T* V = static_cast<const T*>(a.v) + h * DH;
-  __shared__ float Ks[gKey][DH];
-  __shared__ float Vs[gKey][DH];
+  __shared__ __attribute__((aligned(16))) float Ks[KT * LDR], Vs[KT * LDR];
 
-  float q[DH], o[DH];
-  const int64_t qrow = row0 + min(qi, qlen - 1);
+  // four values of a row from head dim d on (zeros past DH)
+  auto load4 = [&](const T* p, int d) {
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    if (DH % 4 == 0 && d >= DH) return v;
+    if constexpr (std::is_same<T, float>::value) {
+      if (vec) return *reinterpret_cast<const f32x4_t*>(p + d);
+    } else {
+      if (vec) {
+        const u32x2_t r = *reinterpret_cast<const u32x2_t*>(p + d);
+        return f32x4_t{__uint_as_float(r[0] << 16), __uint_as_float(r[0] & 0xffff0000u), __uint_as_float(r[1] << 16),
+                       __uint_as_float(r[1] & 0xffff0000u)};
+      }
+    }
 #pragma unroll
-  for (int d = 0; d < DH; ++d) {
-    q[d] = load_f32(Q + qrow * a.ld_q + d);
-    o[d] = 0.f;
+    for (int j = 0; j < 4; ++j) v[j] = load_f32(p + d + j);
+    return v;
+  };
+  f32x4_t qf[ND], o[ND];
+  const T* qrow = Q + (row0 + min(qi, qlen - 1)) * a.ld_q;
+#pragma unroll
+  for (int s = 0; s < ND; ++s) {
+    qf[s] = load4(qrow, 16 * s + 4 * q);
+    o[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   int klo = 0, khi = klen;
   if (a.window > 0) {
     klo = max(0, q0 - a.window);
-    khi = min(klen, q0 + gQ - 1 + a.window + 1);
+    khi = min(klen, q0 + fQ - 1 + a.window + 1);
   }
   const int qlo = a.window > 0 ? max(0, qi - a.window) : 0;
   const int qhi = a.window > 0 ? min(klen, qi + a.window + 1) : klen;
-  float m_i = -INFINITY, l_i = 0.f;
+  float m_i = -INFINITY, l_i = 0.f;  // l_i: this lane's keys only, until the end
 
-  for (int kt = klo; kt < khi; kt += gKey) {
-    for (int idx = tid; idx < gKey * DH; idx += gQ) {
-      const int r = idx / DH, d = idx - r * DH;
-      const int key = min(kt + r, klen - 1);
-      Ks[r][d] = load_f32(K + (row0 + key) * a.ld_k + d);
-      Vs[r][d] = load_f32(V + (row0 + key) * a.ld_v + d);
+  f32x4_t kr[NL], vr[NL];
+  auto fetch = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int idx = min(tid + 256 * i, KT * DP / 4 - 1), r = idx / (DP / 4), d = 4 * (idx - r * (DP / 4));
+      const int64_t row = row0 + min(kt + r, klen - 1);
+      kr[i] = load4(K + row * a.ld_k, d);
+      vr[i] = load4(V + row * a.ld_v, d);
+    }
+  };
+  if (klo < khi) fetch(klo);
+  for (int kt = klo; kt < khi; kt += KT) {
+    __syncthreads();  // the previous tile's reads
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int idx = min(tid + 256 * i, KT * DP / 4 - 1), r = idx / (DP / 4), d = 4 * (idx - r * (DP / 4));
+      *reinterpret_cast<f32x4_t*>(Ks + r * LDR + d) = kr[i];
+      *reinterpret_cast<f32x4_t*>(Vs + r * LDR + d) = vr[i];
     }
     __syncthreads();
-    float sc[gKey];
+    if (kt + KT < khi) fetch(kt + KT);
+    f32x4_t s[NB];
     float tmax = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < gKey; ++j) {
-      const int key = kt + j;
-      float s = 0.f;
+    for (int kb = 0; kb < NB; ++kb) {
+      s[kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int d = 0; d < DH; ++d) s += q[d] * Ks[j][d];
-      s *= a.scale;
-      if (key < qlo || key >= qhi) s = -INFINITY;
-      sc[j] = s;
-      tmax = fmaxf(tmax, s);
+      for (int t = 0; t < ND; ++t) {
+        const f32x4_t kf = *reinterpret_cast<const f32x4_t*>(Ks + (kb * 16 + c) * LDR + 16 * t + 4 * q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j], qf[t][j], s[kb], 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = kt + kb * 16 + 4 * q + e;
+        s[kb][e] = key < qlo || key >= qhi ? -INFINITY : s[kb][e] * a.scale;
+        tmax = fmaxf(tmax, s[kb][e]);
+      }
     }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
     const float m_new = fmaxf(m_i, tmax);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = expf(m_i - m_use);
     m_i = m_new;
     l_i *= alpha;
 #pragma unroll
-    for (int d = 0; d < DH; ++d) o[d] *= alpha;
+    for (int t = 0; t < ND; ++t)
 #pragma unroll
-    for (int j = 0; j < gKey; ++j) {
-      const float p = expf(sc[j] - m_use);
-      l_i += p;
+      for (int e = 0; e < 4; ++e) o[t][e] *= alpha;
 #pragma unroll
-      for (int d = 0; d < DH; ++d) o[d] += p * Vs[j][d];
-    }
-    __syncthreads();
+    for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float p = expf(s[kb][e] - m_use);
+        l_i += p;
+        const float* vrow = Vs + (kb * 16 + 4 * q + e) * LDR + c;
+#pragma unroll
+        for (int t = 0; t < ND; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * t], p, o[t], 0, 0, 0);
+      }
   }
-  if (active) {
-    const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
-    T* O = static_cast<T*>(a.o) + (row0 + qi) * a.ld_o + h * DH;
+  l_i += __shfl_xor(l_i, 16, 64);
+  l_i += __shfl_xor(l_i, 32, 64);
+  if (qi >= qlen) return;
+  const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
+  T* O = static_cast<T*>(a.o) + (row0 + qi) * a.ld_o + h * DH + 4 * q;
 #pragma unroll
-    for (int d = 0; d < DH; ++d) store_f32(O + d, o[d] * inv);
-  }
+  for (int t = 0; t < ND; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (DP == DH || 16 * t + 4 * q + e < DH) store_f32(O + 16 * t + e, o[t][e] * inv);
 }
 
 template <typename T>
-void launch_generic(const AttnArgs& a, hipStream_t st) {
-  dim3 grid((a.max_q + gQ - 1) / gQ, a.H, a.B), block(gQ);
+void launch_f32(const AttnArgs& a, hipStream_t st) {
+  const uintptr_t align = 4 * sizeof(T) - 1;
+  auto ok = [&](const void* p, int64_t ld) { return (reinterpret_cast<uintptr_t>(p) & align) == 0 && ld % 4 == 0; };
+  const int vec = a.Dh % 4 == 0 && ok(a.q, a.ld_q) && ok(a.k, a.ld_k) && ok(a.v, a.ld_v);
+  dim3 grid((a.max_q + fQ - 1) / fQ, a.H, a.B), block(256);
   switch (a.Dh) {
-    case 8: attn_generic_kernel<T, 8><<<grid, block, 0, st>>>(a); break;
-    case 16: attn_generic_kernel<T, 16><<<grid, block, 0, st>>>(a); break;
-    case 32: attn_generic_kernel<T, 32><<<grid, block, 0, st>>>(a); break;
-    case 64: attn_generic_kernel<T, 64><<<grid, block, 0, st>>>(a); break;
-    case 128: attn_generic_kernel<T, 128><<<grid, block, 0, st>>>(a); break;
+    case 8: attn_f32_kernel<T, 8><<<grid, block, 0, st>>>(a, vec); break;
+    case 16: attn_f32_kernel<T, 16><<<grid, block, 0, st>>>(a, vec); break;
+    case 32: attn_f32_kernel<T, 32><<<grid, block, 0, st>>>(a, vec); break;
+    case 64: attn_f32_kernel<T, 64><<<grid, block, 0, st>>>(a, vec); break;
+    case 128: attn_f32_kernel<T, 128><<<grid, block, 0, st>>>(a, vec); break;
     default: fail("attention: head_dim must be 8, 16, 32, 64 or 128");
   }
 }
@@ -914,10 +970,10 @@ void launch_attn(const AttnArgs& a, hipStream_t st) {
   }
   require(!a.q_log2_scaled, "attention: pre-scaled queries need the bf16 head_dim-64 kernel");
   if (a.dtype == DT_BF16)
-    launch_generic<bf16_t>(a, st);
+    launch_f32<bf16_t>(a, st);
   else
-    launch_generic<float>(a, st);
-  check_launch("attn_generic");
+    launch_f32<float>(a, st);
+  check_launch("attn_f32");
 }
 
 namespace {
