@@ -487,35 +487,67 @@ __global__ void gather_rows_kernel(const float* src, int64_t ld_src, const int* 
 // (-1e4 where the marker is padding), their softmax (exp in float, sums in
 // double, as the reference), top1, top1 - top2, the entropy over log(max(2,
 // live markers)) and kf / 255, written after the row's [CLS] hidden state.
-// One workgroup per row; the short serial part runs on one lane.
-__global__ void act_features_kernel(const float* s2, const int* mmask, int K, const float* cls,
+// One workgroup per row.
+constexpr int kActThreads = 256;
+__global__ __launch_bounds__(kActThreads) void act_features_kernel(const float* s2, const int* mmask, int K, const float* cls,
                                     int64_t ld_cls, int D, float* logits, float* ain,
                                     int64_t ld_ain) {
-  const int b = blockIdx.x;
+  const int b = blockIdx.x, tid = threadIdx.x;
   const float* sb = s2 + static_cast<int64_t>(b) * K;
   const int* mb = mmask + static_cast<int64_t>(b) * K;
   float* lg = logits + static_cast<int64_t>(b) * K;
   float* f = ain + static_cast<int64_t>(b) * ld_ain;
-  for (int k = threadIdx.x; k < K; k += blockDim.x) lg[k] = mb[k] ? sb[k] : -1e4f;
-  for (int j = threadIdx.x; j < D; j += blockDim.x) f[j] = cls[static_cast<int64_t>(b) * ld_cls + j];
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  float mx = lg[0];
-  for (int j = 1; j < K; ++j) mx = fmaxf(mx, lg[j]);
-  double s = 0.0;
-  for (int j = 0; j < K; ++j) s += static_cast<double>(expf(lg[j] - mx));
-  double top1 = 0.0, top2 = 0.0, ent = 0.0, ksum = 0.0;
-  for (int j = 0; j < K; ++j) {
-    const double v = static_cast<double>(expf(lg[j] - mx)) / s;
-    if (v > top1) {
-      top2 = top1;
-      top1 = v;
-    } else if (v > top2) {
-      top2 = v;
-    }
-    ent -= v * log(fmax(v, 1e-9));
-    ksum += mb[j];
+  __shared__ float red[kActThreads], ex[kActThreads];
+  __shared__ double pv[kActThreads], pl[kActThreads], total;
+  float mx = -INFINITY;
+  for (int k = tid; k < K; k += kActThreads) {
+    lg[k] = mb[k] ? sb[k] : -1e4f;
+    mx = fmaxf(mx, lg[k]);
   }
+  for (int j = tid; j < D; j += kActThreads) f[j] = cls[static_cast<int64_t>(b) * ld_cls + j];
+  red[tid] = mx;
+  __syncthreads();
+  for (int off = kActThreads / 2; off > 0; off >>= 1) {
+    if (tid < off) red[tid] = fmaxf(red[tid], red[tid + off]);
+    __syncthreads();
+  }
+  mx = red[0];
+  // every thread evaluates its markers' exp, quotient and log; lane 0 adds them
+  // in marker order (11 -> 6.2 us against one lane evaluating all of 16)
+  double s = 0.0;
+  for (int k0 = 0; k0 < K; k0 += kActThreads) {
+    if (k0 + tid < K) ex[tid] = expf(lg[k0 + tid] - mx);
+    __syncthreads();
+    if (tid == 0)
+      for (int j = 0; j < min(kActThreads, K - k0); ++j) s += static_cast<double>(ex[j]);
+    __syncthreads();
+  }
+  if (tid == 0) total = s;
+  __syncthreads();
+  double top1 = 0.0, top2 = 0.0, ent = 0.0, ksum = 0.0;
+  for (int k0 = 0; k0 < K; k0 += kActThreads) {
+    if (k0 + tid < K) {
+      const double v = static_cast<double>(expf(lg[k0 + tid] - mx)) / total;
+      pv[tid] = v;
+      pl[tid] = log(fmax(v, 1e-9));
+      red[tid] = static_cast<float>(mb[k0 + tid]);
+    }
+    __syncthreads();
+    if (tid == 0)
+      for (int j = 0; j < min(kActThreads, K - k0); ++j) {
+        const double v = pv[j];
+        if (v > top1) {
+          top2 = top1;
+          top1 = v;
+        } else if (v > top2) {
+          top2 = v;
+        }
+        ent -= v * pl[j];
+        ksum += red[j];
+      }
+    __syncthreads();
+  }
+  if (tid != 0) return;
   const double kf = fmax(2.0, ksum);
   ent /= log(kf);
   f[D + 0] = static_cast<float>(top1);
@@ -660,7 +692,7 @@ void launch_act_features(const float* s2, const int* mmask, int B, int K, const 
                          int64_t ld_cls, int D, float* logits, float* ain, int64_t ld_ain,
                          hipStream_t st) {
   if (B <= 0 || K <= 0) return;
-  act_features_kernel<<<B, 256, 0, st>>>(s2, mmask, K, cls, ld_cls, D, logits, ain, ld_ain);
+  act_features_kernel<<<B, kActThreads, 0, st>>>(s2, mmask, K, cls, ld_cls, D, logits, ain, ld_ain);
   check_launch("act_features");
 }
 
