@@ -696,8 +696,21 @@ __device__ void attn_item_of(const int32_t* qbp, int Bb, int H, int64_t i, int& 
 // the items of runs x, x + 8, x + 16, ... (runs of kAttnRun items of the
 // batch's item order).  With split, the items of the tail ranks follow the
 // others as half items, both halves of an item side by side.
+// With tok_pos, the Bb workgroups past the list's index the tokens (as
+// launch_token_index): both only read the sequence table, and a launch of its
+// own cost 2-3 us of a call's start.
 __global__ __launch_bounds__(256) void attn_items_kernel(const int32_t* table, int Bb, int H, int n_slots,
-                                                         int split, int32_t* items) {
+                                                         int split, int32_t* items, int* tok_pos, int* tok_seq) {
+  const int list_wgs = (n_slots + 255) / 256;
+  if (static_cast<int>(blockIdx.x) >= list_wgs) {
+    const int b = blockIdx.x - list_wgs;
+    const int s0 = table[kSeqHdr + b], n = table[kSeqHdr + Bb + b];
+    for (int i = threadIdx.x; i < n; i += 256) {
+      tok_pos[s0 + i] = i;
+      tok_seq[s0 + i] = b;
+    }
+    return;
+  }
   const int s = blockIdx.x * 256 + threadIdx.x;
   if (s >= n_slots) return;
   const int32_t* qbp = table + seq_table_qbp(Bb);
@@ -1014,14 +1027,16 @@ int attn_item_slots(int Tb, int Bb, int H, bool split) {
 }
 
 void launch_attn_items(const int32_t* table, int Bb, int H, int n_slots, bool split, int32_t* items,
-                       hipStream_t st) {
+                       int* tok_pos, int* tok_seq, hipStream_t st) {
   if (n_slots <= 0) return;
   require(table && items && (reinterpret_cast<uintptr_t>(items) & 15u) == 0 && Bb >= 1 && H >= 1 &&
               H < 16384 && n_slots % 8 == 0,
           "attention items: bad arguments");
   // (the caller keeps every sequence below 65536 query blocks: the item
   // holds the block index in 16 bits, the head in 14)
-  attn_items_kernel<<<(n_slots + 255) / 256, 256, 0, st>>>(table, Bb, H, n_slots, split ? 1 : 0, items);
+  require(!tok_pos == !tok_seq, "attention items: both token arrays or neither");
+  attn_items_kernel<<<(n_slots + 255) / 256 + (tok_pos ? Bb : 0), 256, 0, st>>>(table, Bb, H, n_slots, split ? 1 : 0,
+                                                                               items, tok_pos, tok_seq);
   check_launch("attn_items");
 }
 

@@ -920,7 +920,6 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
   void* O = w.O;
   void* G = w.G;
 
-  launch_token_index(seq_start, q_len, Bb, w.tok_pos, w.tok_seq, st);
   // the attention work list of the batch, when the bf16 head_dim-64 kernel runs
   // (the list holds a query block's index in 16 bits); the shortest
   // sequences' items split by keys when the batch may hold such (launch_attn_items)
@@ -931,7 +930,9 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
   if (attn_list) {
     require(attn_slots <= w.attn_slots_cap && attn_pairs <= w.attn_pairs_cap,
             "attention work list: workspace too small");
-    launch_attn_items(si, Bb, H_, attn_slots, attn_split, w.attn_items, st);
+    launch_attn_items(si, Bb, H_, attn_slots, attn_split, w.attn_items, w.tok_pos, w.tok_seq, st);
+  } else {
+    launch_token_index(seq_start, q_len, Bb, w.tok_pos, w.tok_seq, st);
   }
   // short batches: attention folds the output projection in (AttnArgs::wo),
   // each head's partial product going to the split-K workspace, and the

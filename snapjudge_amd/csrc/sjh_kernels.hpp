@@ -281,9 +281,10 @@ int attn_split_pairs(int Tb, int Bb, int H);
 // Ints of the list: n_slots int4 items, then (split) one pair index per slot.
 inline size_t attn_items_ints(int n_slots) { return 5u * static_cast<size_t>(n_slots); }
 // Fills items[0, n_slots) (and the pair indices when split) from the sequence
-// table (its query-block prefix).
+// table (its query-block prefix), and with tok_pos and tok_seq the token index
+// (launch_token_index) of the table's sequences.
 void launch_attn_items(const int32_t* table, int Bb, int H, int n_slots, bool split, int32_t* items,
-                       hipStream_t st);
+                       int* tok_pos, int* tok_seq, hipStream_t st);
 // Output rows of the split items: O = (2^(m1-M) O1 + 2^(m2-M) O2) /
 // (2^(m1-M) l1 + 2^(m2-M) l2), M = max(m1, m2), bf16 into o (row stride ld_o,
 // head h at column 64 h).  Workgroups past the batch's pairs return.
