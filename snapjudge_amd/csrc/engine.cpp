@@ -1550,8 +1550,6 @@ size_t Engine::scratch_layout(const BatchPlan& p, Ws& ws) const {
   };
   const size_t seq = take(seq_table_ints(p.Bb) * 4);
   const size_t tok_pos = take(t * 4), tok_seq = take(t * 4);
-  const bool shortb = short_batch(p.Tb);
-  const size_t X = take(shortb ? t * D * 4 : 0);
   const size_t Y = take(t * D * as), QKV = take(t * 3 * D * as), O = take(t * D * as);
   const size_t G = take(t * static_cast<size_t>(F_) * as);
   const size_t Z = lora_r_ > 0 ? take(t * static_cast<size_t>(lora_r_) * 4) : 0;
@@ -1561,10 +1559,14 @@ size_t Engine::scratch_layout(const BatchPlan& p, Ws& ws) const {
   const size_t items = take(static_cast<size_t>(n_items) * 16);
   ws = Ws();
   if (off > kScratchBytes) return off;
+  // a short batch's residual stream, last and only where it still fits: without
+  // it the batch runs on the caller's rows, through the general GEMMs (same bits)
+  const bool in_ws = short_batch(p.Tb) && off + align256(t * D * 4) <= kScratchBytes;
+  const size_t X = take(in_ws ? t * D * 4 : 0);
   ws.seq = reinterpret_cast<int32_t*>(scratch_ + seq);
   ws.tok_pos = reinterpret_cast<int*>(scratch_ + tok_pos);
   ws.tok_seq = reinterpret_cast<int*>(scratch_ + tok_seq);
-  ws.X = shortb ? reinterpret_cast<float*>(scratch_ + X) : nullptr;
+  ws.X = in_ws ? reinterpret_cast<float*>(scratch_ + X) : nullptr;
   ws.Y = scratch_ + Y;
   ws.QKV = scratch_ + QKV;
   ws.O = scratch_ + O;

@@ -64,3 +64,23 @@ def test_short_fp8_rows(orc, D, lens):
         assert float(np.abs(p - r).max()) <= 5e-3
     assert float(np.abs(act - ra).max()) <= 5e-3
     m.close()
+
+
+def test_short_batch_beside_a_full_scratch_array():
+    # 256 rows of this width leave no room for the residual stream in the fixed
+    # array: the batch still runs there, on the caller's rows, with the same bits
+    rl, enc, w = synth.make_model(hidden_size=1664, num_hidden_layers=1, num_attention_heads=26,
+                                  intermediate_size=1024, vocab_size=512, store="BF16", seed=23)
+    m = sj.Model(w, synth.flat_cfg(rl, enc), precision=sj.SJH_PREC_BF16)
+    for lens in ([256], [100, 41]):
+        ids, _, n = synth.batch_with_lens(lens, max(lens), 512, seed=8)
+        print(f"full scratch array lens={lens}", flush=True)
+        d_ids = torch.from_numpy(np.concatenate([ids[b, :k] for b, k in enumerate(lens)]).astype(np.int32)).cuda()
+        outs = []
+        for fn in (m.encode_device, m.encode_device_noalloc):
+            out = torch.full((sum(lens), 1664), float("nan"), dtype=torch.float32, device="cuda")
+            fn(d_ids.data_ptr(), np.asarray(lens, np.int32), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            outs.append(out.cpu().numpy())
+        assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
+    m.close()
