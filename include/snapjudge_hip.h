@@ -110,9 +110,10 @@ typedef struct sjh_options {
                          hidden size a multiple of 256 up to 1024, one round of at least
                          128 tiles), its epilogue also writes the LayerNorm that reads the
                          residual stream next; 0: that LayerNorm runs as a launch of its
-                         own; 2: as 1 with any number of tiles, and a tile waits for its panel's other tiles for one poll only, so that
-                         most tiles take the path of a tile that gave up waiting (the
-                         results are the same bits as with 1; for tests) */
+                         own; 2: as 1 with any number of tiles, and a tile waits for its
+                         panel's other tiles for one poll only, so that most tiles take
+                         the path of a tile that gave up waiting (the results are the
+                         same bits as with 1; for tests) */
   int32_t fuse_attn_wo; /* 1 (default): on short batches (at most 256 tokens, bf16, head_dim
                          64) attention also multiplies each head's output by its slice of
                          Wo, and the LayerNorm that reads the residual stream next adds the

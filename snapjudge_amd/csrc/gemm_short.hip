@@ -424,6 +424,7 @@ bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p
 
 bool gemm_short_ok(const GemmArgs& g) {
   const bool w8 = g.w_dtype == DT_FP8;
+  if (g.ln_stats_in || g.ln_y || g.rln_y) return false;  // (no LayerNorm in these epilogues)
   if (g.M <= 0 || g.M % 32 != 0 || g.M > kShortMaxRows || g.M_dev || g.N < 2 || g.N % 2 != 0 || g.K <= 0 || g.K % 64 != 0)
     return false;
   if (g.in_dtype != DT_BF16 || !g.A || !aligned(g.A, 16) || g.lda % 8 != 0 || g.lda < g.K || g.lda >= (int64_t{1} << 28))
