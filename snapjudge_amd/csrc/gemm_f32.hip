@@ -9,8 +9,9 @@
 // 16x16x4 block takes 32 cycles), so operand bandwidth is not the limit once
 // the loads are coalesced.
 //  - gemm_f32_staged_kernel: 64x64 or 32x64 tiles, four waves, 32-deep K steps
-//    moved by direct-to-LDS loads (eight lanes take 128 contiguous bytes of a
-//    row) through a three-stage ring.
+//    in which eight lanes take 32 consecutive values of a row, moved by
+//    direct-to-LDS loads through a three-stage ring, or through registers for
+//    bf16 operands, rows no vector load can read and K of a few steps.
 //  - gemm_f32_split_kernel, for products too small to give every CU such a
 //    tile: 16x64 or 16x16 tiles whose eight waves each take an eighth of K and
 //    add their sums through LDS in wave order, so that the weights stream
@@ -25,6 +26,8 @@
 // of 96 questions, 1536 x 768 x 768, 85 (mean) -> 30 us (60 TFLOP/s; 8192 x
 // 3072 x 768 reaches 107 of the 154 that a large fp32 product of the vendor
 // library does); QKV of 569 rows 112 -> 32 us, the residual products 107 -> 21.
+// Through registers: bf16 8000 x 768 x 777 304 -> 110 us (the split kernel 573),
+// fp32 2000 x 768 x 769 126 -> 35, and 20000 x 768 x 8, a LoRA update, 36 -> 30.
 // Both take the k values of a 16-deep group in the lanes' own order: lane
 // (r, q) holds row r's values 4 q + [0, 4) and MFMA j of the group takes the
 // lanes' j-th values, the same k on both sides.  The epilogue runs on the fp32
@@ -236,18 +239,21 @@ __global__ __launch_bounds__(64 * WGK) void gemm_f32_split_kernel(GemmArgs g0, i
   tile_epilogue<BM, BN, NT, OutT>(Cs, LDC, m0, tile_n, g);
 }
 
-// BM x 64 tiles of fp32 operands, four waves in 2 x 2.  vec: 16-byte aligned
-// rows; otherwise, and for the last partial K step, rows are staged value by
-// value.
-template <typename OutT, int BM>
+// BM x 64 tiles, four waves in 2 x 2.  DIRECT (fp32, 16-byte aligned rows): whole
+// K steps go straight to LDS, two ahead of their use.  Otherwise, and for the
+// last partial step, a step's values pass through registers (widened there, the
+// next step's in flight meanwhile) into one LDS buffer; vec: rows aligned to four
+// values, which one load then takes.
+template <typename InT, typename OutT, int BM, bool DIRECT>
 __global__ __launch_bounds__(256) void gemm_f32_staged_kernel(GemmArgs g0, int vec) {
+  static_assert(!DIRECT || std::is_same<InT, float>::value, "direct loads move fp32 rows");
   GemmArgs g = g0;
   if (g.M_dev) g.M = *g.M_dev;
-  constexpr int BN = 64, BK = 32, NS = 3, RB = BK * 4, ROWS = BM + BN, LDC = BN + 4;
+  constexpr int BN = 64, BK = 32, NS = DIRECT ? 3 : 1, RB = BK * 4, ROWS = BM + BN, LDC = BN + 4;
   constexpr int TI = BM / 32, TJ = 2, G = ROWS / 32;  // load instructions (8 rows each) per wave and stage
   constexpr int STAGE = ROWS * RB;
-  static_assert(NS * STAGE >= BM * LDC * 4, "the epilogue's tile reuses the ring");
-  __shared__ __attribute__((aligned(16))) char ring[NS * STAGE];
+  constexpr int LDS = NS * STAGE > BM * LDC * 4 ? NS * STAGE : BM * LDC * 4;  // the epilogue's tile reuses the ring
+  __shared__ __attribute__((aligned(16))) char ring[LDS];
   int tile_m, tile_n;
   pick_tile<BM, BN>(g, g0.M, tile_m, tile_n);
   const int m0 = tile_m * BM;
@@ -255,25 +261,14 @@ __global__ __launch_bounds__(256) void gemm_f32_staged_kernel(GemmArgs g0, int v
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, q = lane >> 4;
-  const float* A = static_cast<const float*>(g.A);
-  const float* W = static_cast<const float*>(g.W);
+  const InT* A = static_cast<const InT*>(g.A);
+  const InT* W = static_cast<const InT*>(g.W);
   auto row_ptr = [&](int r) {
     return r < BM ? A + static_cast<int64_t>(min(m0 + r, g.M - 1)) * g.lda : W + w_row<BN>(g, tile_n, r - BM) * g.ldw;
   };
   // 16-byte chunk c of row r sits at slot c ^ swz(r): 16 consecutive rows at one
   // chunk then fall into 16 different 16-byte bank groups
   auto swz = [](int r) { return (r >> 1) & 7; };
-  const float* src[G];
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    const int r = 8 * (wave + 4 * i) + (lane >> 3);
-    src[i] = row_ptr(r) + 4 * ((lane & 7) ^ swz(r));
-  }
-  auto issue = [&](int kt, int slot) {
-#pragma unroll
-    for (int i = 0; i < G; ++i) load_lds16(src[i] + kt * BK, ring + slot * STAGE + (wave + 4 * i) * 1024);
-  };
-
   f32x4_t acc[TI][TJ];
 #pragma unroll
   for (int i = 0; i < TI; ++i)
@@ -301,31 +296,70 @@ __global__ __launch_bounds__(256) void gemm_f32_staged_kernel(GemmArgs g0, int v
     }
   };
 
-  const int nk = vec ? g.K / BK : 0;
+  int k0 = 0;
+  if constexpr (DIRECT) {
+    const float* src[G];
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < nk) issue(s, s);
-  int slot = 0;
-  for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk)
-      wait_vmcnt<G*(NS - 2)>();
-    else
-      wait_vmcnt<0>();
-    wait_lgkm0();  // this wave's reads of the slot that is refilled next
-    __builtin_amdgcn_s_barrier();
-    if (kt + NS - 1 < nk) issue(kt + NS - 1, slot == 0 ? NS - 1 : slot - 1);
-    compute(slot);
-    slot = slot + 1 == NS ? 0 : slot + 1;
-  }
-  for (int k0 = nk * BK; k0 < g.K; k0 += BK) {
-    __syncthreads();
-    for (int idx = tid; idx < ROWS * 8; idx += 256) {
-      const int r = idx >> 3, c = idx & 7;
-      const f32x4_t v = load4_upto(row_ptr(r) + k0 + 4 * c, g.K - k0 - 4 * c);
-      *reinterpret_cast<f32x4_t*>(ring + r * RB + (c ^ swz(r)) * 16) = v;
+    for (int i = 0; i < G; ++i) {
+      const int r = 8 * (wave + 4 * i) + (lane >> 3);
+      src[i] = row_ptr(r) + 4 * ((lane & 7) ^ swz(r));
     }
-    __syncthreads();
-    compute(0);
+    auto issue = [&](int kt, int slot) {
+#pragma unroll
+      for (int i = 0; i < G; ++i) load_lds16(src[i] + kt * BK, ring + slot * STAGE + (wave + 4 * i) * 1024);
+    };
+    const int nk = g.K / BK;
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s)
+      if (s < nk) issue(s, s);
+    int slot = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+      if (kt + 1 < nk)
+        wait_vmcnt<G*(NS - 2)>();
+      else
+        wait_vmcnt<0>();
+      wait_lgkm0();  // this wave's reads of the slot that is refilled next
+      __builtin_amdgcn_s_barrier();
+      if (kt + NS - 1 < nk) issue(kt + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+      compute(slot);
+      slot = slot + 1 == NS ? 0 : slot + 1;
+    }
+    k0 = nk * BK;
+  }
+  if (k0 < g.K) {
+    constexpr int NP = ROWS * 8 / 256;  // four-value pieces per thread and step
+    const int c = tid & 7;
+    const InT* row[NP];
+    f32x4_t v[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) row[i] = row_ptr((tid >> 3) + 32 * i) + 4 * c;
+    auto fetch = [&](int k) {
+      const int left = g.K - k - 4 * c;  // k values of this thread's four that exist
+      if (left < 4) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) v[i] = load4_upto(row[i] + k, left);
+      } else if (vec) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) v[i] = load4(row[i] + k);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[i][j] = load_f32(row[i] + k + j);
+      }
+    };
+    fetch(k0);
+    for (; k0 < g.K; k0 += BK) {
+      __syncthreads();  // the reads of the step before
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const int r = (tid >> 3) + 32 * i;
+        *reinterpret_cast<f32x4_t*>(ring + r * RB + (c ^ swz(r)) * 16) = v[i];
+      }
+      __syncthreads();
+      if (k0 + BK < g.K) fetch(k0 + BK);
+      compute(0);
+    }
   }
   __syncthreads();
   float* Cs = reinterpret_cast<float*>(ring);
@@ -347,6 +381,14 @@ unsigned tiles_of(const GemmArgs& g, int BM, int BN) {
   return static_cast<unsigned>(tiles);
 }
 
+template <typename InT, typename OutT, bool DIRECT>
+void launch_staged(const GemmArgs& g, int vec, unsigned t32, hipStream_t st) {
+  if (t32 >= 2048)
+    gemm_f32_staged_kernel<InT, OutT, 64, DIRECT><<<tiles_of(g, 64, 64), 256, 0, st>>>(g, vec);
+  else
+    gemm_f32_staged_kernel<InT, OutT, 32, DIRECT><<<t32, 256, 0, st>>>(g, vec);
+}
+
 template <typename InT, typename OutT>
 void launch_typed(const GemmArgs& g, hipStream_t st) {
   const uintptr_t align = 4 * sizeof(InT) - 1;
@@ -357,11 +399,19 @@ void launch_typed(const GemmArgs& g, hipStream_t st) {
   // several rounds of them anyway (fewer operand bytes per product), 32 below,
   // so that the last round is shorter.
   const unsigned t32 = tiles_of(g, 32, 64);
-  if (std::is_same<InT, float>::value && t32 >= 192) {
-    if (t32 >= 2048)
-      gemm_f32_staged_kernel<OutT, 64><<<tiles_of(g, 64, 64), 256, 0, st>>>(g, vec);
-    else
-      gemm_f32_staged_kernel<OutT, 32><<<t32, 256, 0, st>>>(g, vec);
+  if (t32 >= 192) {
+    // direct-to-LDS steps where rows allow them and there are enough steps to
+    // pay for the ring: with several rounds of tiles its 48 KB leave three
+    // workgroups on a CU instead of eight to cover each other's start and
+    // epilogue (18432 x 3072 x 256: 323 us direct, 289 through registers; 8192 x
+    // 768 at K = 384 55.5 and 55.8, 512 66.9 and 68.9).  One round has no such
+    // cover to lose (1000 x 768 x 64 6.5 and 7.0, 768 20.6 and 22.0).  The same bits.
+    if constexpr (std::is_same<InT, float>::value)
+      if (vec && g.K >= (t32 >= 2048 ? 384 : 64)) {
+        launch_staged<InT, OutT, true>(g, vec, t32, st);
+        return;
+      }
+    launch_staged<InT, OutT, false>(g, vec, t32, st);
     return;
   }
   // 16x16 tiles where 16x64 ones would leave CUs idle and the epilogue (bias,

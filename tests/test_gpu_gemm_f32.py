@@ -61,3 +61,24 @@ def test_gemm_f32_geglu_pairs(M, F, K):
     lim = 1.13 * e[:, :F] * np.abs(u[:, F:]) + np.abs(u[:, :F]) * e[:, F:] + e[:, :F] * e[:, F:]
     lim += 8 * 2.0 ** -24 * (np.abs(u[:, :F]) + 1) * (np.abs(u[:, F:]) + 1)  # erff, its argument, the products
     assert np.all(np.abs(out.cpu().numpy() - act * u[:, F:]) <= lim)
+
+
+# 32- and 64-row tiles staged through registers: rows no vector load can read,
+# steps ending inside a piece of four values, K of less than a step, bf16 rows
+# (products exact in fp32; a bf16 store rounds by at most 2^-8 of its value)
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(300, 1500, 51), (257, 1601, 772), (2100, 2050, 16), (2049, 2111, 3), (2100, 2050, 70)])
+def test_gemm_f32_staged_through_registers(M, N, K, dtype):
+    print(f"gemm staged {dtype} M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + 5 * N + K)
+    td, code = (torch.bfloat16, sj.SJH_BF16) if dtype == "bf16" else (torch.float32, sj.SJH_F32)
+    A, W = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(td) for s in ((M, K), (N, K)))
+    a, w, b = A.double().numpy(), W.double().numpy(), rng.standard_normal(N).astype(np.float32)
+    A, W, B = A.cuda(), W.cuda(), torch.from_numpy(b).cuda()
+    out = torch.full((M + 1, N), 7.0, device="cuda", dtype=td)
+    sj.check(sj.lib().sjh_gemm(P(A), P(W), P(B), P(out), M, N, K, 0, code, None))
+    got, ref = out.cpu().double().numpy(), a @ w.T + b
+    lim = bound(a, w, K, b[None] + 0 * ref) + (2.0 ** -8 * np.abs(ref) if dtype == "bf16" else 0)
+    lim *= 1 + 2.0 ** -8  # the store rounds the computed value, not the exact one
+    assert np.all(np.abs(got[:M] - ref) <= lim)
+    assert np.all(got[M] == 7.0)
