@@ -828,10 +828,12 @@ std::vector<std::tuple<const char*, double, int64_t>> Engine::profile_totals() {
 }
 
 namespace {
-// Launches g on the short-batch kernels where they take it.
-bool try_gemm_short(const GemmArgs& g0, hipStream_t st) {
+// Launches g on the short-batch kernels where they take it.  They need no row
+// count where every row of the launch exists: in the workspace, so for all
+// outputs but a residual stream that is the caller's.
+bool try_gemm_short(const GemmArgs& g0, const Ws& w, hipStream_t st) {
   GemmArgs g = g0;
-  g.M_dev = nullptr;
+  if (g.epi != EPI_RESID || g.X == w.X) g.M_dev = nullptr;
   if (!gemm_short_ok(g)) return false;
   launch_gemm_short(g, st);
   return true;
@@ -843,7 +845,7 @@ void Engine::gemm(const char* name, const GemmArgs& g0, const Ws& w, hipStream_t
   g.partial = w.partial;
   g.partial_cap = w.partial_cap;
   prof_begin(st);
-  if (!short_rows || !try_gemm_short(g, st)) launch_gemm(g, st);
+  if (!short_rows || !try_gemm_short(g, w, st)) launch_gemm(g, st);
   prof_end(name, st);
 }
 
@@ -861,7 +863,7 @@ void Engine::resid_gemm_ln(const char* gname, const GemmArgs& g0, const char* ln
   folded.xio = g.X;
   folded.n_parts = 1;
   prof_begin(st);
-  const bool done = short_rows && try_gemm_short(g, st);
+  const bool done = short_rows && try_gemm_short(g, w, st);
   const int S = !done && g.M <= 256 && ln_takes_parts(folded) ? launch_gemm_resid_partials(g, st) : 0;
   if (!done && S == 0) launch_gemm(g, st);
   prof_end(gname, st);
@@ -942,11 +944,11 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
                        D % kAttnWoCols == 0 && D <= 1024 && w.partial &&
                        static_cast<int64_t>(H_) * T * D <= w.partial_cap;
 
-  // a short batch's residual stream stays in the workspace (all Tb rows); the
-  // final norm writes the caller's rows
-  const bool shortb = w.X && short_batch(T);
+  // a short batch's residual stream stays in the workspace (all Tb rows), where
+  // that has room for it; the final norm writes the caller's rows
+  const bool shortb = short_batch(T), own_x = shortb && w.X;
   float* const out = X;
-  if (shortb) X = w.X;
+  if (own_x) X = w.X;
 
   // src/model.cpp:332-340: X = LN(emb[ids]); layer 0 reads X itself.  BERT
   // family (src/sj_model.cpp:220-237): X = LN(word[ids] + pos[position] ; w, b)
@@ -1000,7 +1002,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
     a.y_dtype = adt;
     a.ld_y = D;
     a.M = T;
-    a.M_dev = shortb ? nullptr : T_dev;  // (all rows exist: nothing waits for the row count)
+    a.M_dev = own_x ? nullptr : T_dev;  // (all rows exist: nothing waits for the row count)
     a.D = D;
     return a;
   };
@@ -1154,7 +1156,7 @@ void Engine::enqueue_encoder(const BatchPlan& p, const Ws& w, const int32_t* d_i
       a.y_dtype = adt;
       a.ld_y = D;
       a.M = T;
-      a.M_dev = shortb ? nullptr : T_dev;
+      a.M_dev = own_x ? nullptr : T_dev;
       a.D = D;
       if (attn_wo) {  // attention wrote the heads' partials of O . Wo^T
         LnArgs f = a;
@@ -1560,7 +1562,7 @@ size_t Engine::scratch_layout(const BatchPlan& p, Ws& ws) const {
   ws = Ws();
   if (off > kScratchBytes) return off;
   // a short batch's residual stream, last and only where it still fits: without
-  // it the batch runs on the caller's rows, through the general GEMMs (same bits)
+  // it the batch runs on the caller's rows (same bits)
   const bool in_ws = short_batch(p.Tb) && off + align256(t * D * 4) <= kScratchBytes;
   const size_t X = take(in_ws ? t * D * 4 : 0);
   ws.seq = reinterpret_cast<int32_t*>(scratch_ + seq);

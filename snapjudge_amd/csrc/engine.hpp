@@ -93,7 +93,7 @@ struct Ws {
   int32_t* seq = nullptr;  // sequence table (sjh_kernels.hpp, seq_table_ints(Bb) ints)
   int* tok_pos = nullptr;  // [Tb] position of each token in its sequence
   int* tok_seq = nullptr;  // [Tb] sequence of each token
-  float* X = nullptr;  // [Tb, D] residual stream of a short batch (Engine::short_batch), or none
+  float* X = nullptr;  // [Tb, D] residual stream of a short batch (Engine::short_batch); none: the caller's rows
   void *Y = nullptr, *QKV = nullptr, *O = nullptr, *G = nullptr;
   float* Z = nullptr;  // LoRA [Tb, r]
   float* partial = nullptr;  // split-K partial sums
@@ -206,17 +206,17 @@ class Engine {
   void end_call(hipStream_t st);
 
   // launch helpers (record profile events when enabled)
-  // (short_rows: the launch's rows all exist, so that the short-batch kernels
-  // of gemm_short.hip may run where they take the product)
+  // (short_rows: a short batch, whose products take the kernels of gemm_short.hip
+  // where those cover them)
   void gemm(const char* name, const GemmArgs& g, const Ws& w, hipStream_t st, bool short_rows = false);
   void ln(const char* name, const LnArgs& a, hipStream_t st);
   // X += A . W^T followed by the layer norm `a` that reads X: for short
   // batches the split-K residual epilogue is folded into that layer norm.
   void resid_gemm_ln(const char* gname, const GemmArgs& g, const char* lname, LnArgs a,
                      const Ws& w, hipStream_t st, bool short_rows);
-  // Whether a batch launched for Tb rows keeps its residual stream in the
-  // workspace (Ws::X), whose rows reach the launch's, so that its products may
-  // take the short-batch kernels
+  // Whether the products of a batch launched for Tb rows may take the short-batch
+  // kernels.  Its residual stream stays in the workspace (Ws::X) where that has
+  // room for it, so that every row of a launch exists
   bool short_batch(int Tb) const { return act_dt_ == DT_BF16 && Tb <= kShortMaxRows; }
   // Sets g up to finish the LayerNorm a (of X's rows into bf16 Y) in its
   // residual epilogue (GemmArgs::rln_y) and returns true where that applies;

@@ -10,7 +10,8 @@
 //  - what the epilogue reads (RoPE rows, the residual stream) is loaded with
 //    them, not after the products;
 //  - no kernel reads the batch's row count first: every row of the launch is
-//    computed (the buffers hold them), whatever is in the surplus ones;
+//    computed (the buffers hold them), whatever is in the surplus ones (but for a
+//    residual stream in the caller's memory, whose rows end with the batch);
 //  - residual products cut K over the waves of one workgroup and add the
 //    slices there, in slice order, so that no partial sums travel through
 //    memory to the LayerNorm that would add them.
@@ -309,8 +310,10 @@ __global__ __launch_bounds__(1024) void gemm_short_resid_kernel(GemmArgs g) {
   const int u0 = wave * C, nu = min(C, units - u0);  // >= 1
 
   // the residual stream's two columns of this thread's item
+  // (rows past a device row count do not exist: the last one's are read again)
   const int er = (tid & 255) / 8, en = tile_n * BN + 2 * (tid & 7);
-  float* xp = g.X + static_cast<int64_t>(m0 + er) * g.ldx + min(en, g.N - 2);
+  const int rows = g.M_dev ? *g.M_dev : g.M;
+  float* xp = g.X + static_cast<int64_t>(min(m0 + er, rows - 1)) * g.ldx + min(en, g.N - 2);
   const f32x2_t x = *reinterpret_cast<const f32x2_t*>(xp);
 
   u32x4_t av[C][4], wv[C][W8 ? 1 : 2];
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(1024) void gemm_short_resid_kernel(GemmArgs g) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) P[(t * 16 + 4 * q + e) * LDC + r16] = acc[t][e];
   __syncthreads();
-  if (tid < 256 && en < g.N) {
+  if (tid < 256 && en < g.N && m0 + er < rows) {
     f32x2_t v = {0.f, 0.f};
     const char* p = lds + (er * LDC + 2 * (tid & 7)) * 4;
     for (int s = 0; s < slices; ++s) {
@@ -425,7 +428,8 @@ bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p
 bool gemm_short_ok(const GemmArgs& g) {
   const bool w8 = g.w_dtype == DT_FP8;
   if (g.ln_stats_in || g.ln_y || g.rln_y) return false;  // (no LayerNorm in these epilogues)
-  if (g.M <= 0 || g.M % 32 != 0 || g.M > kShortMaxRows || g.M_dev || g.N < 2 || g.N % 2 != 0 || g.K <= 0 || g.K % 64 != 0)
+  if (g.M_dev && g.epi != EPI_RESID) return false;
+  if (g.M <= 0 || g.M % 32 != 0 || g.M > kShortMaxRows || g.N < 2 || g.N % 2 != 0 || g.K <= 0 || g.K % 64 != 0)
     return false;
   if (g.in_dtype != DT_BF16 || !g.A || !aligned(g.A, 16) || g.lda % 8 != 0 || g.lda < g.K || g.lda >= (int64_t{1} << 28))
     return false;

@@ -116,7 +116,8 @@ void launch_gemm(const GemmArgs& g, hipStream_t st);
 // products (bias, activation; K a multiple of 256 up to 1024, bf16 output) and
 // residual products (K a multiple of 64), bf16 rows and bf16 or fp8 weights, a
 // multiple of 32 rows up to kShortMaxRows.  All M rows of the launch are read
-// and written (no M_dev): the buffers hold them.
+// and written (no M_dev): the buffers hold them, but for the rows of X of a
+// residual product with M_dev.
 constexpr int kShortMaxRows = 256;
 // The K slices of a residual product of a short batch: slices of chunk 64-deep
 // units each (the last may be shorter).

@@ -66,21 +66,25 @@ def test_short_fp8_rows(orc, D, lens):
     m.close()
 
 
-def test_short_batch_beside_a_full_scratch_array():
+@pytest.mark.parametrize("prec", [sj.SJH_PREC_BF16, sj.SJH_PREC_FP8W])
+def test_short_batch_beside_a_full_scratch_array(prec):
     # 256 rows of this width leave no room for the residual stream in the fixed
     # array: the batch still runs there, on the caller's rows, with the same bits
+    # (fp8 weights too: its residual products keep their K slices); rows past the
+    # batch, of which a launch has some, are not the caller's
     rl, enc, w = synth.make_model(hidden_size=1664, num_hidden_layers=1, num_attention_heads=26,
                                   intermediate_size=1024, vocab_size=512, store="BF16", seed=23)
-    m = sj.Model(w, synth.flat_cfg(rl, enc), precision=sj.SJH_PREC_BF16)
-    for lens in ([256], [100, 41]):
+    m = sj.Model(w, synth.flat_cfg(rl, enc), precision=prec)
+    for lens in ([256], [150, 101], [100, 41]):
         ids, _, n = synth.batch_with_lens(lens, max(lens), 512, seed=8)
-        print(f"full scratch array lens={lens}", flush=True)
+        print(f"full scratch array prec={prec} lens={lens}", flush=True)
         d_ids = torch.from_numpy(np.concatenate([ids[b, :k] for b, k in enumerate(lens)]).astype(np.int32)).cuda()
         outs = []
         for fn in (m.encode_device, m.encode_device_noalloc):
-            out = torch.full((sum(lens), 1664), float("nan"), dtype=torch.float32, device="cuda")
+            out = torch.full((sum(lens) + 64, 1664), float("nan"), dtype=torch.float32, device="cuda")
             fn(d_ids.data_ptr(), np.asarray(lens, np.int32), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
             torch.cuda.synchronize()
-            outs.append(out.cpu().numpy())
+            assert bool(torch.isnan(out[sum(lens):]).all())
+            outs.append(out[:sum(lens)].cpu().numpy())
         assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
     m.close()

@@ -30,7 +30,7 @@ def run(m, fn, ids, lens, D, stream):
     return out.cpu().numpy()
 
 
-@pytest.mark.parametrize("prec", [sj.SJH_PREC_BF16, sj.SJH_PREC_FP32])
+@pytest.mark.parametrize("prec", [sj.SJH_PREC_BF16, sj.SJH_PREC_FP32, sj.SJH_PREC_FP8W])
 def test_noalloc_equals_encode_device(prec):
     import torch
 
@@ -39,8 +39,8 @@ def test_noalloc_equals_encode_device(prec):
     D, V = cfg["hidden_size"], cfg["vocab_size"]
     m = sj.Model(w, cfg, precision=prec)
     stream = torch.cuda.current_stream().cuda_stream
-    # ~1900 tokens (bf16) / ~850 tokens (fp32: twice the bytes per token)
-    big = (synth.make_batch(6, 400, 100, 400, V, seed=82) if prec == sj.SJH_PREC_BF16
+    # ~1900 tokens (bf16 rows) / ~850 tokens (fp32: twice the bytes per token)
+    big = (synth.make_batch(6, 400, 100, 400, V, seed=82) if prec != sj.SJH_PREC_FP32
            else synth.make_batch(4, 300, 100, 300, V, seed=82))
     small = synth.make_batch(2, 120, 40, 120, V, seed=83)   # <= 256 tokens: split-K residuals
     for name, (ids, _, lens) in (("big", big), ("small", small)):
