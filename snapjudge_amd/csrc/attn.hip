@@ -851,7 +851,9 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a, int vec) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int idx = min(tid + 256 * i, KT * DP / 4 - 1), r = idx / (DP / 4), d = 4 * (idx - r * (DP / 4));
-      const int64_t row = row0 + min(kt + r, klen - 1);
+      // (keys past khi repeat the last one: a row outside the window of every query
+      // here must not come in with weight 0, which an infinite V value makes NaN)
+      const int64_t row = row0 + min(kt + r, khi - 1);
       kr[i] = load4(K + row * a.ld_k, d);
       vr[i] = load4(V + row * a.ld_v, d);
     }

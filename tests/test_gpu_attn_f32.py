@@ -52,3 +52,28 @@ def test_attn_f32_edges(Dh, L, window, dtype):
             ds = (Dh + 3) * u * scale * (np.abs(q) @ np.abs(k).T).max(1)[~dead]
             lim = (2 * (2 * ds + (n + 8) * u) * np.abs(v).max())[:, None] + (2.0 ** -8 * np.abs(want) if dtype == "bf16" else 0)
             assert np.all(np.abs(got[b, ~dead, h] - want) <= lim), (b, h)
+
+
+@pytest.mark.parametrize("key", [72, 90, 135, 150, 170, 199])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attn_f32_infinite_rows_past_the_window(key, bad):
+    # an infinite or NaN V row reaches the queries of a 64-query block that has it
+    # in some query's window, and no others: their values are as without it
+    print(f"attn f32 V row {key} {bad}", flush=True)
+    L, H, Dh, window = 200, 2, 64, 8
+    g = torch.Generator(device="cuda").manual_seed(key)
+    qkv = torch.randn(1, L, 3, H, Dh, generator=g, device="cuda")
+    dl = torch.tensor([L], dtype=torch.int32, device="cuda")
+    P = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    outs = []
+    for v in (None, bad):
+        if v is not None:
+            qkv[0, key, 2] = v
+        out = torch.full((L, H * Dh), 7.0, device="cuda")
+        sj.check(sj.lib().sjh_attn(P(qkv), P(dl), P(out), 1, L, H, Dh, window, sj.SJH_F32, None))
+        outs.append(out.cpu())
+    block = torch.arange(L) // 64 * 64
+    free = (key < block - window) | (key >= block + 64 + window)
+    seen = (torch.arange(L) - key).abs() <= window
+    assert torch.equal(outs[1][free], outs[0][free])
+    assert not torch.isfinite(outs[1][seen]).any()
