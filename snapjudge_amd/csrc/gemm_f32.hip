@@ -131,14 +131,21 @@ __device__ __forceinline__ f32x4_t load4_upto(const T* p, int n) {
   return v;
 }
 
-// Tile of workgroup blockIdx.x.  XCDs get contiguous runs of tiles (workgroups
-// go round-robin over the 8 XCDs); the operand with fewer rows is the one that
-// every XCD reads whole.
+// Workgroups of a grid's row: a grid dimension holds fewer than 2^32 threads
+// (512 of them here at most), so that more tiles take several rows.
+constexpr unsigned kGridX = 1u << 22;
+
+// Tile of this workgroup, or false past the last one.  XCDs get contiguous runs
+// of tiles (workgroups go round-robin over the 8 XCDs); the operand with fewer
+// rows is the one that every XCD reads whole.
 template <int BM, int BN>
-__device__ __forceinline__ void pick_tile(const GemmArgs& g, int launch_m, int& tile_m, int& tile_n) {
+__device__ __forceinline__ bool pick_tile(const GemmArgs& g, int launch_m, int& tile_m, int& tile_n) {
   const int tiles_n = g.epi == EPI_GEGLU ? (g.N + BN / 2 - 1) / (BN / 2) : (g.N + BN - 1) / BN;
   const int tiles_m = (launch_m + BM - 1) / BM;
-  const int nb = static_cast<int>(gridDim.x), bid = static_cast<int>(blockIdx.x);
+  const int nb = tiles_m * tiles_n;
+  const unsigned wg = blockIdx.y * kGridX + blockIdx.x;
+  if (wg >= static_cast<unsigned>(nb)) return false;
+  const int bid = static_cast<int>(wg);
   const int xcd = bid & 7, per = nb >> 3, rem = nb & 7;
   const int tile = xcd * per + min(xcd, rem) + (bid >> 3);
   if (launch_m < g.N) {
@@ -148,6 +155,7 @@ __device__ __forceinline__ void pick_tile(const GemmArgs& g, int launch_m, int& 
     tile_m = tile / tiles_n;
     tile_n = tile - tile_m * tiles_n;
   }
+  return true;
 }
 
 // 16 x 16 TJ tiles, K cut into WGK slices of whole 16-deep steps, one wave
@@ -160,7 +168,7 @@ __global__ __launch_bounds__(64 * WGK) void gemm_f32_split_kernel(GemmArgs g0, i
   constexpr int BM = 16, BN = 16 * TJ, NT = 64 * WGK, LDC = BN + 4;
   __shared__ float Cs[WGK * BM * LDC];
   int tile_m, tile_n;
-  pick_tile<BM, BN>(g, g0.M, tile_m, tile_n);
+  if (!pick_tile<BM, BN>(g, g0.M, tile_m, tile_n)) return;  // (uniform)
   const int m0 = tile_m * BM;
   if (m0 >= g.M) return;  // a row tile past the device row count (uniform)
 
@@ -255,7 +263,7 @@ __global__ __launch_bounds__(256) void gemm_f32_staged_kernel(GemmArgs g0, int v
   constexpr int LDS = NS * STAGE > BM * LDC * 4 ? NS * STAGE : BM * LDC * 4;  // the epilogue's tile reuses the ring
   __shared__ __attribute__((aligned(16))) char ring[LDS];
   int tile_m, tile_n;
-  pick_tile<BM, BN>(g, g0.M, tile_m, tile_n);
+  if (!pick_tile<BM, BN>(g, g0.M, tile_m, tile_n)) return;  // (uniform)
   const int m0 = tile_m * BM;
   if (m0 >= g.M) return;  // a row tile past the device row count (uniform)
 
@@ -381,12 +389,14 @@ unsigned tiles_of(const GemmArgs& g, int BM, int BN) {
   return static_cast<unsigned>(tiles);
 }
 
+dim3 grid_of(unsigned tiles) { return dim3(std::min(tiles, kGridX), (tiles + kGridX - 1) / kGridX); }
+
 template <typename InT, typename OutT, bool DIRECT>
 void launch_staged(const GemmArgs& g, int vec, unsigned t32, hipStream_t st) {
   if (t32 >= 2048)
-    gemm_f32_staged_kernel<InT, OutT, 64, DIRECT><<<tiles_of(g, 64, 64), 256, 0, st>>>(g, vec);
+    gemm_f32_staged_kernel<InT, OutT, 64, DIRECT><<<grid_of(tiles_of(g, 64, 64)), 256, 0, st>>>(g, vec);
   else
-    gemm_f32_staged_kernel<InT, OutT, 32, DIRECT><<<t32, 256, 0, st>>>(g, vec);
+    gemm_f32_staged_kernel<InT, OutT, 32, DIRECT><<<grid_of(t32), 256, 0, st>>>(g, vec);
 }
 
 template <typename InT, typename OutT>
@@ -418,9 +428,9 @@ void launch_typed(const GemmArgs& g, hipStream_t st) {
   // activation, residual) needs no pairs of columns
   const int vec_steps = vec ? g.K / 16 : 0;
   if (tiles_of(g, 16, 64) < 256 && (g.epi == EPI_STORE || g.epi == EPI_RESID))
-    gemm_f32_split_kernel<InT, OutT, 1, 8, 6><<<tiles_of(g, 16, 16), 512, 0, st>>>(g, vec_steps);
+    gemm_f32_split_kernel<InT, OutT, 1, 8, 6><<<grid_of(tiles_of(g, 16, 16)), 512, 0, st>>>(g, vec_steps);
   else
-    gemm_f32_split_kernel<InT, OutT, 4, 8, 6><<<tiles_of(g, 16, 64), 512, 0, st>>>(g, vec_steps);
+    gemm_f32_split_kernel<InT, OutT, 4, 8, 6><<<grid_of(tiles_of(g, 16, 64)), 512, 0, st>>>(g, vec_steps);
 }
 
 }  // namespace

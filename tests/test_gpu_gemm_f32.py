@@ -82,3 +82,22 @@ def test_gemm_f32_staged_through_registers(M, N, K, dtype):
     lim *= 1 + 2.0 ** -8  # the store rounds the computed value, not the exact one
     assert np.all(np.abs(got[:M] - ref) <= lim)
     assert np.all(got[M] == 7.0)
+
+
+def test_gemm_f32_more_tiles_than_one_grid_dimension_holds():
+    # 2^24 tiles of 256 threads: gelu(x) * y of one product each, so that every
+    # value is known; the output is 33 GB
+    M, F = 65, 1 << 28
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 60 GB of free device memory")
+    print(f"geglu M={M} F={F} K=1", flush=True)
+    A = torch.ones(M, 1, dtype=torch.bfloat16, device="cuda")
+    A[-1] = 2
+    W = torch.ones(2 * F, 1, dtype=torch.bfloat16, device="cuda")
+    out = torch.zeros(M, F, dtype=torch.bfloat16, device="cuda")
+    sj.check(sj.lib().sjh_gemm_geglu(P(A), P(W), P(out), M, F, 1, sj.SJH_BF16, None))
+    for r in (0, 1, 31, 32, 63, 64):
+        x = 2.0 if r == M - 1 else 1.0
+        want = x * 0.5 * x * (1 + float(torch.erf(torch.tensor(x / 2 ** 0.5, dtype=torch.float64))))
+        lo, hi = float(out[r].min()), float(out[r].max())
+        assert lo == hi and abs(lo - want) <= 2.0 ** -8 * want, r
