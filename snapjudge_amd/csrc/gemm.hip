@@ -96,8 +96,10 @@ __device__ __forceinline__ float swap16(float v, bool hi_row) {
 
 // Epilogue on the accumulators in registers (see the comment above).
 // TAB_LDS: the RoPE table rows of the tile are staged in LDS at rope_tab
-// (given whenever the tile has rotated columns).
-template <int BM, int BN, int WM, int WN, int TI, int TJ, int EPI, typename OutT, bool TAB_LDS = false>
+// (given whenever the tile has rotated columns).  PERS: the persistent kernel,
+// whose 128 registers a wave leave no room for the rows that a partial tile
+// takes together in the others (3 to 48 of them went to memory).
+template <int BM, int BN, int WM, int WN, int TI, int TJ, int EPI, typename OutT, bool TAB_LDS = false, bool PERS = false>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)[TI][TJ], int m0,
                                               int tile_n, int wm, int wn, int l32, int hb,
                                               const char* rope_tab = nullptr) {
@@ -167,6 +169,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
 #pragma unroll
     for (int j = 0; j < TJ; ++j) bv[j] = g.bias ? g.bias[min(c0 + j * 32 + l32, g.N - 1)] : 0.f;
     auto body = [&](auto checked) {  // checked: the wave's rows or columns run past M or N
+      constexpr bool kClamp = decltype(checked)::value && !PERS;
       auto in = [&](int r, int j) {
         if constexpr (decltype(checked)::value)
           return rw + r + 4 * hb < g.M && c0 + j * 32 + l32 < g.N;
@@ -184,16 +187,16 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
             // a partial tile reads its last row and column again rather than
             // branch per element (a branch would wait for each load)
             const float* xc = nullptr;
-            if constexpr (decltype(checked)::value) xc = g.X + static_cast<int64_t>(min(rw + r + 4 * hb, g.M - 1)) * g.ldx;
+            if constexpr (kClamp) xc = g.X + static_cast<int64_t>(min(rw + r + 4 * hb, g.M - 1)) * g.ldx;
 #pragma unroll
             for (int j = 0; j < TJ; ++j) {
-              if constexpr (decltype(checked)::value)
+              if constexpr (kClamp)
                 xv[e][j] = xc[min(c0 + j * 32 + l32, g.N - 1)];
               else
-                xv[e][j] = *reinterpret_cast<const float*>(xr + j * 128);
+                xv[e][j] = in(r, j) ? *reinterpret_cast<const float*>(xr + j * 128) : 0.f;
             }
           }
-          if constexpr (decltype(checked)::value) {
+          if constexpr (kClamp) {
 #pragma unroll
             for (int e = 0; e < RG; ++e)
 #pragma unroll
@@ -355,29 +358,39 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
     for (int j = 0; j < TJ; ++j) bv[j] = g.bias ? g.bias[min(c0 + j * 32 + l32, g.N - 1)] : 0.f;
     auto body = [&](auto checked, auto act_tag) {
       constexpr int ACT = decltype(act_tag)::value;
+      // a partial tile: eight rows' values, then their stores (see GEGLU); a full
+      // one row by row (3072 x 3072 x 768 GELU 29.8 us, 30.4 by eights)
+      constexpr int RG = decltype(checked)::value && !PERS ? 8 : 1;
+      auto value = [&](int i, int j, int e) {
+        const float v = acc[i][j][e] + bv[j];
+        if constexpr (ACT == 1)
+          return gelu_out<OutT>(v);
+        else if constexpr (ACT == 2)
+          return fmaxf(v, 0.f);
+        else
+          return v;
+      };
 #pragma unroll
       for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int e0 = 0; e0 < 16; e0 += 8) {
-          float v[8][TJ];  // eight rows' values, then their stores (see GEGLU)
+        for (int e0 = 0; e0 < 16; e0 += RG) {
+          float v[RG][TJ];
+          if constexpr (RG > 1) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
+            for (int e = 0; e < RG; ++e)
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-              v[e][j] = acc[i][j][e0 + e] + bv[j];
-              if constexpr (ACT == 1)
-                v[e][j] = gelu_out<OutT>(v[e][j]);
-              else if constexpr (ACT == 2)
-                v[e][j] = fmaxf(v[e][j], 0.f);
-            }
+              for (int j = 0; j < TJ; ++j) v[e][j] = value(i, j, e0 + e);
+          }
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
+          for (int e = 0; e < RG; ++e) {
             const int r = i * 32 + 8 * ((e0 + e) >> 2) + ((e0 + e) & 3);
+            if (decltype(checked)::value && rw + r + 4 * hb >= g.M) continue;
             char* orow = const_cast<char*>(ow) + static_cast<uint32_t>(r * ldb + lo);
 #pragma unroll
-            for (int j = 0; j < TJ; ++j)
-              if (!decltype(checked)::value || (rw + r + 4 * hb < g.M && c0 + j * 32 + l32 < g.N))
-                store_f32(reinterpret_cast<OutT*>(orow + j * 32 * EB), v[e][j]);
+            for (int j = 0; j < TJ; ++j) {
+              if (decltype(checked)::value && c0 + j * 32 + l32 >= g.N) continue;
+              store_f32(reinterpret_cast<OutT*>(orow + j * 32 * EB), RG > 1 ? v[e][j] : value(i, j, e0 + e));
+            }
           }
         }
     };
@@ -972,12 +985,17 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_dma_kernel(GemmArgs 
   // RPI * q + lane / CPR into chunk slot lane % CPR, reading the logical
   // chunk that the swizzle maps there
   // (fp8 W rows: 16 rows of 64 bytes per instruction, four lanes each)
+  // Row groups counted in a scalar register cost instructions before the first
+  // load: without, 512 x 768 x 768 takes 7.6 us (7.7), 3000 x 1152 GEGLU x 768 17.8
+  // (18.2); but the deep 128x128 ring is the faster with them (2304 x 1024 x 2624
+  // 26.8 us, 28.1 without), and fp8 rows need a uniform choice of the operand.
+  constexpr bool kUniWave = W8 || (BM == 128 && BN == 128 && NS == 4);
   const char* src[G];
   bool w8_src[G];  // uniform: a source that advances BK bytes per step, not 2 BK
   const int lrow = lane / CPR, cslot = lane % CPR;
 #pragma unroll
   for (int i = 0; i < G; ++i) {
-    const int q = __builtin_amdgcn_readfirstlane(wave) + TT::NW * i;
+    const int q = (kUniWave ? __builtin_amdgcn_readfirstlane(wave) : wave) + TT::NW * i;
     w8_src[i] = W8 && q >= BM / TT::RPI;
     if (w8_src[i]) {
       const int r = (q - BM / TT::RPI) * 16 + (lane >> 2);
@@ -1768,7 +1786,7 @@ void gemm_bf16_pers_kernel(GemmArgs g0) {
     if constexpr (kSwap)
       pers_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT>(g, acc, m0, tn, wme, wne, l32e, hbe);
     else
-      gemm_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT, kRopeLds>(g, acc, m0, tn, wme, wne, l32e, hbe,
+      gemm_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT, kRopeLds, true>(g, acc, m0, tn, wme, wne, l32e, hbe,
                                                                rope_tab);
   }
 }
