@@ -1791,18 +1791,6 @@ void gemm_bf16_pers_kernel(GemmArgs g0) {
   }
 }
 
-int num_cus() {
-  static int n = 0;
-  if (n == 0) {
-    int dev = 0, v = 0;
-    hip_check(hipGetDevice(&dev), "gemm: hipGetDevice");
-    hip_check(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev),
-              "gemm: CU count");
-    n = v > 0 ? v : 256;
-  }
-  return n;
-}
-
 // Output tiles of BM rows by BN rows of W.
 int64_t count_tiles(const GemmArgs& g, int BM, int BN) {
   const int n = g.epi == EPI_GEGLU ? BN / 2 : BN;
@@ -1969,22 +1957,32 @@ bool pers_ok(const GemmArgs& g) {
 //          residual 18.0 (the persistent kernel's 72 tiles 28.5); plain and GEGLU
 //          products keep four waves of 64x64 (1501 x 3072 x 768 GELU 18.1, eight
 //          waves 18.6)
-//  TPERS   the persistent 256x256 kernel from kPersMinTiles tiles on: 3072 x 2624
-//          GEGLU x 1024 (246 tiles) 35.0 (T128 40.6), 18 432 x 2304 x 768 72.8
-//          (88); 3072 x 3072 x 1024 (144 tiles) 30.8 against 29.8
+//  TPERS   the persistent 256x256 kernel, once the 128x128 tiles no longer run all
+//          at once (the few of a second round cost as much as the first), on all of
+//          the CUs or not: 9216 x 1024 x 2624 residual (576 of them, 144 of 256x256)
+//          59.6 (T128 71.6), 9216 x 1024 x 4096 81 (102), 4096 x 2304 x 768 RoPE 24.1
+//          (26.1); 8192 x 1024 x 4096 (512) 81.1 against 62.6.  Short K loops, whose
+//          time is the epilogue's, need 5 / 8 of the CUs: 9216 x 1024 x 256 (144)
+//          12.9 against 11.7, 6144 x 1536 x 512 (144) 17.4-18.8 against 17.5-17.9; and
+//          with fp8 weights, whose decode two workgroups share a CU's pipes for, those
+//          of up to 1024 do: 3072 x 3072 x 768 GELU (144) 28.4 against 26.3, 9216 x 1024
+//          x 4096 (144) 81.5 against 86.0
 enum Tile { T64, T128x64, T128D, T128, TPERS };
-constexpr int kPersMinTiles = 160;
-// a residual product that also finishes the LayerNorm saves its launch: 12 000 x
-// 768 x (768 / 1152) (141 tiles) 42.5 us with it, 43.5 on T128 and two launches
-constexpr int kRlnMinTiles = 128;
+// A residual product that also finishes the LayerNorm saves its launch, on half the
+// CUs or more: 12 000 x 768 x (768 / 1152) (141 tiles) 42.5 us with it, 43.5 on T128
+// and two launches.
+bool rln_pays(int64_t tiles) { return 2 * tiles >= num_cus(); }
 
 Tile pick_tile(const GemmArgs& g) {
   if (g.rln_y || g.ln_y || g.ln_stats_in) return TPERS;  // (checked by launch_gemm)
   const int cus = num_cus();
   if (count_tiles(g, 64, 64) <= cus) return T64;
   if (count_tiles(g, 128, 64) <= cus) return T128x64;
-  if (count_tiles(g, 256, 256) >= kPersMinTiles && pers_ok(g)) return TPERS;
-  return count_tiles(g, 128, 128) <= cus ? T128D : T128;
+  const int64_t t128 = count_tiles(g, 128, 128);
+  if (t128 <= cus) return T128D;
+  const int short_k = g.w_dtype == DT_FP8 ? 1024 : g.epi == EPI_STORE ? 512 : 256;
+  if (t128 <= 2 * cus || (g.K <= short_k && 8 * count_tiles(g, 256, 256) < 5 * cus) || !pers_ok(g)) return T128;
+  return TPERS;
 }
 
 template <bool W8>
@@ -2142,6 +2140,17 @@ bool launch_splitk(const GemmArgs& g0, hipStream_t st) {
 
 }  // namespace
 
+// Compute units of the process's (first) device.
+int num_cus() {
+  static const int n = [] {
+    int dev = 0, v = 0;
+    hip_check(hipGetDevice(&dev), "gemm: hipGetDevice");
+    hip_check(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev), "gemm: CU count");
+    return v > 0 ? v : 256;
+  }();
+  return n;
+}
+
 // The bf16 MFMA kernels' operand requirements.
 bool mfma_ok(const GemmArgs& g) {
   return g.in_dtype == DT_BF16 && g.w_dtype == DT_BF16 && g.K % kBK == 0 && g.lda % 8 == 0 &&
@@ -2165,7 +2174,7 @@ bool gemm_takes_rln(const GemmArgs& g, bool any_tiles) {
   if (!(mfma_ok(g) && g.M >= 4096 && pers_ok(g))) return false;
   // one round: every tile a workgroup of its own, all resident at once
   const int64_t tiles = static_cast<int64_t>(g.N / kLnBlock) * ((g.M + 255) / 256);
-  return (any_tiles || tiles >= kRlnMinTiles) &&
+  return (any_tiles || rln_pays(tiles)) &&
          tiles <= static_cast<int64_t>(pers_occupancy<SJH_GEMM_PERS, false>()) * num_cus();
 }
 

@@ -112,6 +112,9 @@ constexpr int kLnBlock = 256;
 constexpr bool kLnFoldEnabled = false;
 constexpr int kLnMaxBlocks = 4;  // D <= 1024 (c1 rows hold 8 bf16, blocks past 4 zero)
 void launch_gemm(const GemmArgs& g, hipStream_t st);
+// Compute units of the device: launches choose their kernel by how many of its
+// tiles they have per CU.
+int num_cus();
 // The short-batch kernels (gemm_short.hip): QKV + RoPE, Wi + GEGLU and plain
 // products (bias, activation; K a multiple of 256 up to 1024, bf16 output) and
 // residual products (K a multiple of 64), bf16 rows and bf16 or fp8 weights, a

@@ -17,14 +17,16 @@ def P(t):
 
 
 # rows of a 1024-column product on 256 CUs: 64x64 tiles up to 1024, 128x64 up to
-# 2048, 128x128 one per CU up to 4096, two per CU, the persistent kernel from 9985
-MS = [9985, 1, 70, 1024, 1025, 2048, 2111, 4033, 4161, 9900]
+# 2048, 128x128 one per CU up to 4096, two per CU; the persistent kernel from 9985
+# (K 192) or as soon as two 128x128 tiles per CU are full, from 8193 (K 1088)
+MS = [9985, 1, 70, 1024, 1025, 2048, 2111, 4033, 4161, 8192, 8193, 9900]
 
 
+@pytest.mark.parametrize("K", [192, 1088])
 @pytest.mark.parametrize("kind", ["store", "geglu", "resid", "rope", "fp8"])
-def test_tile_shapes_give_the_same_bits(kind):
-    print(f"tiles {kind}", flush=True)
-    N, K, H = 1024, 192, 16
+def test_tile_shapes_give_the_same_bits(kind, K):
+    print(f"tiles {kind} K={K}", flush=True)
+    N, H = 1024, 16
     g = torch.Generator(device="cuda").manual_seed(7)
     A = torch.randn(MS[0], K, generator=g, device="cuda").bfloat16()
     nw = {"geglu": 2 * N, "rope": 3 * N}.get(kind, N)
