@@ -393,7 +393,7 @@ dim3 grid_of(unsigned tiles) { return dim3(std::min(tiles, kGridX), (tiles + kGr
 
 template <typename InT, typename OutT, bool DIRECT>
 void launch_staged(const GemmArgs& g, int vec, unsigned t32, hipStream_t st) {
-  if (t32 >= 2048)
+  if (t32 >= 8 * static_cast<unsigned>(num_cus()))
     gemm_f32_staged_kernel<InT, OutT, 64, DIRECT><<<grid_of(tiles_of(g, 64, 64)), 256, 0, st>>>(g, vec);
   else
     gemm_f32_staged_kernel<InT, OutT, 32, DIRECT><<<grid_of(t32), 256, 0, st>>>(g, vec);
@@ -408,8 +408,8 @@ void launch_typed(const GemmArgs& g, hipStream_t st) {
   // rows: 21 us a product against 28 split); 64 rows each where there are
   // several rounds of them anyway (fewer operand bytes per product), 32 below,
   // so that the last round is shorter.
-  const unsigned t32 = tiles_of(g, 32, 64);
-  if (t32 >= 192) {
+  const unsigned t32 = tiles_of(g, 32, 64), cus = static_cast<unsigned>(num_cus());
+  if (t32 >= 3 * cus / 4) {
     // direct-to-LDS steps where rows allow them and there are enough steps to
     // pay for the ring: with several rounds of tiles its 48 KB leave three
     // workgroups on a CU instead of eight to cover each other's start and
@@ -417,7 +417,7 @@ void launch_typed(const GemmArgs& g, hipStream_t st) {
     // 768 at K = 384 55.5 and 55.8, 512 66.9 and 68.9).  One round has no such
     // cover to lose (1000 x 768 x 64 6.5 and 7.0, 768 20.6 and 22.0).  The same bits.
     if constexpr (std::is_same<InT, float>::value)
-      if (vec && g.K >= (t32 >= 2048 ? 384 : 64)) {
+      if (vec && g.K >= (t32 >= 8 * cus ? 384 : 64)) {
         launch_staged<InT, OutT, true>(g, vec, t32, st);
         return;
       }
@@ -427,7 +427,7 @@ void launch_typed(const GemmArgs& g, hipStream_t st) {
   // 16x16 tiles where 16x64 ones would leave CUs idle and the epilogue (bias,
   // activation, residual) needs no pairs of columns
   const int vec_steps = vec ? g.K / 16 : 0;
-  if (tiles_of(g, 16, 64) < 256 && (g.epi == EPI_STORE || g.epi == EPI_RESID))
+  if (tiles_of(g, 16, 64) < cus && (g.epi == EPI_STORE || g.epi == EPI_RESID))
     gemm_f32_split_kernel<InT, OutT, 1, 8, 6><<<grid_of(tiles_of(g, 16, 16)), 512, 0, st>>>(g, vec_steps);
   else
     gemm_f32_split_kernel<InT, OutT, 4, 8, 6><<<grid_of(tiles_of(g, 16, 64)), 512, 0, st>>>(g, vec_steps);

@@ -287,7 +287,7 @@ void launch_plain(const GemmArgs& g, hipStream_t st) {
   // its own; else half the ring, so that two tiles share a CU (128 rows, 288
   // tiles: QKV 5.4 us, against 6.3 with 64-row tiles of the whole K)
   const int tiles_n = g.epi == EPI_GEGLU ? (g.N + 15) / 16 : (g.N + 31) / 32;
-  if (tiles_n * (g.M / 32) <= 256)
+  if (tiles_n * (g.M / 32) <= num_cus())
     launch_k<32, 4, W8>(g, st);
   else
     launch_k<32, 2, W8>(g, st);
