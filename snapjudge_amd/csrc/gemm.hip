@@ -96,10 +96,8 @@ __device__ __forceinline__ float swap16(float v, bool hi_row) {
 
 // Epilogue on the accumulators in registers (see the comment above).
 // TAB_LDS: the RoPE table rows of the tile are staged in LDS at rope_tab
-// (given whenever the tile has rotated columns).  PERS: the persistent kernel,
-// whose 128 registers a wave leave no room for the rows that a partial tile
-// takes together in the others (3 to 48 of them went to memory).
-template <int BM, int BN, int WM, int WN, int TI, int TJ, int EPI, typename OutT, bool TAB_LDS = false, bool PERS = false>
+// (given whenever the tile has rotated columns).
+template <int BM, int BN, int WM, int WN, int TI, int TJ, int EPI, typename OutT, bool TAB_LDS = false>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)[TI][TJ], int m0,
                                               int tile_n, int wm, int wn, int l32, int hb,
                                               const char* rope_tab = nullptr) {
@@ -169,7 +167,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
 #pragma unroll
     for (int j = 0; j < TJ; ++j) bv[j] = g.bias ? g.bias[min(c0 + j * 32 + l32, g.N - 1)] : 0.f;
     auto body = [&](auto checked) {  // checked: the wave's rows or columns run past M or N
-      constexpr bool kClamp = decltype(checked)::value && !PERS;
       auto in = [&](int r, int j) {
         if constexpr (decltype(checked)::value)
           return rw + r + 4 * hb < g.M && c0 + j * 32 + l32 < g.N;
@@ -187,16 +184,16 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
             // a partial tile reads its last row and column again rather than
             // branch per element (a branch would wait for each load)
             const float* xc = nullptr;
-            if constexpr (kClamp) xc = g.X + static_cast<int64_t>(min(rw + r + 4 * hb, g.M - 1)) * g.ldx;
+            if constexpr (decltype(checked)::value) xc = g.X + static_cast<int64_t>(min(rw + r + 4 * hb, g.M - 1)) * g.ldx;
 #pragma unroll
             for (int j = 0; j < TJ; ++j) {
-              if constexpr (kClamp)
+              if constexpr (decltype(checked)::value)
                 xv[e][j] = xc[min(c0 + j * 32 + l32, g.N - 1)];
               else
-                xv[e][j] = in(r, j) ? *reinterpret_cast<const float*>(xr + j * 128) : 0.f;
+                xv[e][j] = *reinterpret_cast<const float*>(xr + j * 128);
             }
           }
-          if constexpr (kClamp) {
+          if constexpr (decltype(checked)::value) {
 #pragma unroll
             for (int e = 0; e < RG; ++e)
 #pragma unroll
@@ -360,7 +357,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
       constexpr int ACT = decltype(act_tag)::value;
       // a partial tile: eight rows' values, then their stores (see GEGLU); a full
       // one row by row (3072 x 3072 x 768 GELU 29.8 us, 30.4 by eights)
-      constexpr int RG = decltype(checked)::value && !PERS ? 8 : 1;
+      constexpr int RG = decltype(checked)::value ? 8 : 1;
       auto value = [&](int i, int j, int e) {
         const float v = acc[i][j][e] + bv[j];
         if constexpr (ACT == 1)
@@ -384,13 +381,11 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
 #pragma unroll
           for (int e = 0; e < RG; ++e) {
             const int r = i * 32 + 8 * ((e0 + e) >> 2) + ((e0 + e) & 3);
-            if (decltype(checked)::value && rw + r + 4 * hb >= g.M) continue;
             char* orow = const_cast<char*>(ow) + static_cast<uint32_t>(r * ldb + lo);
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-              if (decltype(checked)::value && c0 + j * 32 + l32 >= g.N) continue;
-              store_f32(reinterpret_cast<OutT*>(orow + j * 32 * EB), RG > 1 ? v[e][j] : value(i, j, e0 + e));
-            }
+            for (int j = 0; j < TJ; ++j)
+              if (!decltype(checked)::value || (rw + r + 4 * hb < g.M && c0 + j * 32 + l32 < g.N))
+                store_f32(reinterpret_cast<OutT*>(orow + j * 32 * EB), RG > 1 ? v[e][j] : value(i, j, e0 + e));
           }
         }
     };
@@ -1786,7 +1781,7 @@ void gemm_bf16_pers_kernel(GemmArgs g0) {
     if constexpr (kSwap)
       pers_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT>(g, acc, m0, tn, wme, wne, l32e, hbe);
     else
-      gemm_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT, kRopeLds, true>(g, acc, m0, tn, wme, wne, l32e, hbe,
+      gemm_epilogue<BM, BN, TT::WM, TT::WN, TI, TJ, EPI, OutT, kRopeLds>(g, acc, m0, tn, wme, wne, l32e, hbe,
                                                                rope_tab);
   }
 }
