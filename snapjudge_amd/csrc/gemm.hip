@@ -1824,15 +1824,13 @@ void launch_pers_kernel(const GemmArgs& g, hipStream_t st) {
 
 template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8>
 void launch_pers(const GemmArgs& g, hipStream_t st) {
-  const bool bf = g.out_dtype == DT_BF16;
   // a folded LayerNorm's consumer: bf16 outputs of the QKV and GEGLU products
   const bool lni = g.ln_stats_in != nullptr;
-  require(!lni || (bf && (g.epi == EPI_ROPE || g.epi == EPI_GEGLU)),
-          "gemm: a folded LayerNorm's consumer is a bf16 RoPE or GEGLU product");
+  require(!lni || g.epi == EPI_ROPE || g.epi == EPI_GEGLU,
+          "gemm: a folded LayerNorm's consumer is a RoPE or GEGLU product");
   switch (g.epi) {
     case EPI_STORE:
-      bf ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_STORE, bf16_t, 0>(g, st)
-         : launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_STORE, float, 0>(g, st);
+      launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_STORE, bf16_t, 0>(g, st);
       break;
     case EPI_RESID:
       if constexpr (!W8 && BM == 256 && BN == 256 && WGM == 4 && WGN == 4) {
@@ -1846,14 +1844,12 @@ void launch_pers(const GemmArgs& g, hipStream_t st) {
              : launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_RESID, float, 0>(g, st);
       break;
     case EPI_ROPE:
-      lni  ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_ROPE, bf16_t, 1>(g, st)
-      : bf ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_ROPE, bf16_t, 0>(g, st)
-           : launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_ROPE, float, 0>(g, st);
+      lni ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_ROPE, bf16_t, 1>(g, st)
+          : launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_ROPE, bf16_t, 0>(g, st);
       break;
     default:
-      lni  ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_GEGLU, bf16_t, 1>(g, st)
-      : bf ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_GEGLU, bf16_t, 0>(g, st)
-           : launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_GEGLU, float, 0>(g, st);
+      lni ? launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_GEGLU, bf16_t, 1>(g, st)
+          : launch_pers_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI_GEGLU, bf16_t, 0>(g, st);
       break;
   }
 }
@@ -1877,10 +1873,7 @@ void launch_mfma_tile(const GemmArgs& g, hipStream_t st) {
   const int64_t tiles = count_tiles(g, BM, BN);
   require(tiles < (int64_t{1} << 31), "gemm: too many tiles");
   dim3 grid(static_cast<unsigned>(tiles));
-  if (g.out_dtype == DT_BF16 || EPI == EPI_RESID)
-    launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI, bf16_t>(g, grid, st);
-  else
-    launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI, float>(g, grid, st);
+  launch_mfma_kernel<BM, BN, WGM, WGN, NS, BK, W8, EPI, bf16_t>(g, grid, st);
 }
 
 template <int BM, int BN, int WGM, int WGN, int NS, int BK, bool W8>
@@ -2074,9 +2067,7 @@ constexpr int kSkBM = 128, kSkBN = 64;
 template <int EPI>
 void launch_splitk_epi(const GemmArgs& g, dim3 grid, hipStream_t st) {
   constexpr int lds = 2 * DTile<kSkBM, kSkBN, 2, 2, 2, 64>::STAGE_BYTES;
-  auto kern = g.out_dtype == DT_BF16 || EPI == EPI_RESID
-                  ? gemm_bf16_dma_kernel<kSkBM, kSkBN, 2, 2, 2, 64, EPI, bf16_t, true>
-                  : gemm_bf16_dma_kernel<kSkBM, kSkBN, 2, 2, 2, 64, EPI, float, true>;
+  auto kern = gemm_bf16_dma_kernel<kSkBM, kSkBN, 2, 2, 2, 64, EPI, bf16_t, true>;
   kern<<<grid, 256, lds, st>>>(g);
 }
 
@@ -2125,10 +2116,7 @@ bool launch_splitk(const GemmArgs& g0, hipStream_t st) {
   if (S == 0) return false;
   const int64_t outs = static_cast<int64_t>(g.M) * g.N;
   dim3 eg(static_cast<unsigned>((outs + 255) / 256));
-  if (g.out_dtype == DT_BF16 || g.epi == EPI_RESID)
-    splitk_epilogue_kernel<bf16_t><<<eg, 256, 0, st>>>(g, S);
-  else
-    splitk_epilogue_kernel<float><<<eg, 256, 0, st>>>(g, S);
+  splitk_epilogue_kernel<bf16_t><<<eg, 256, 0, st>>>(g, S);
   check_launch("gemm_splitk_epilogue");
   return true;
 }
@@ -2146,9 +2134,10 @@ int num_cus() {
   return n;
 }
 
-// The bf16 MFMA kernels' operand requirements.
+// The bf16 MFMA kernels' operand requirements; their outputs are bf16 rows or the
+// fp32 residual stream (fp32 outputs of bf16 operands go to gemm_f32.hip).
 bool mfma_ok(const GemmArgs& g) {
-  return g.in_dtype == DT_BF16 && g.w_dtype == DT_BF16 && g.K % kBK == 0 && g.lda % 8 == 0 &&
+  return (g.out_dtype == DT_BF16 || g.epi == EPI_RESID) && g.in_dtype == DT_BF16 && g.w_dtype == DT_BF16 && g.K % kBK == 0 && g.lda % 8 == 0 &&
          g.ldw % 8 == 0 && aligned16(g.A) && aligned16(g.W) &&
          (g.epi != EPI_ROPE || g.head_dim == 64) && (g.epi != EPI_GEGLU || g.N % 64 == 0);
 }
@@ -2227,7 +2216,8 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   }
   if (g.w_dtype == DT_FP8) {
     // fp8 weights: 16-byte chunks of the codes' rows
-    require(g.in_dtype == DT_BF16, "gemm: fp8 weights need bf16 activations");
+    require(g.in_dtype == DT_BF16 && (g.out_dtype == DT_BF16 || g.epi == EPI_RESID),
+            "gemm: fp8 weights need bf16 activations and outputs");
     require(g.w_scale && aligned16(g.w_scale), "gemm: fp8 weights need per-row scales");
     require(g.K % 64 == 0 && g.lda % 8 == 0 && g.ldw % 16 == 0 && aligned16(g.A) &&
                 aligned16(g.W),
@@ -2242,8 +2232,8 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     return;
   }
   require(g.w_dtype == DT_BF16 || g.w_dtype == DT_F32, "gemm: unknown weight type");
-  const bool mfma = g.in_dtype == DT_BF16 && g.K % kBK == 0 && g.lda % 8 == 0 &&
-                    g.ldw % 8 == 0 && aligned16(g.A) && aligned16(g.W) &&
+  const bool mfma = g.in_dtype == DT_BF16 && (g.out_dtype == DT_BF16 || g.epi == EPI_RESID) &&
+                    g.K % kBK == 0 && g.lda % 8 == 0 && g.ldw % 8 == 0 && aligned16(g.A) && aligned16(g.W) &&
                     (g.epi != EPI_ROPE || g.head_dim == 64) &&
                     (g.epi != EPI_GEGLU || g.N % 64 == 0);
   if (g.epi == EPI_ROPE && !mfma)
