@@ -7,8 +7,9 @@
 // fixed cost of a few microseconds.  So:
 //  - as many of a tile's loads as fit are in flight at once, issued by four
 //    waves (or one wave per K slice) before the first use;
-//  - what the epilogue reads (RoPE rows, the residual stream) is loaded with
-//    them, not after the products;
+//  - the RoPE rows and the residual stream that an epilogue reads are loaded
+//    with them, not after the products (the bias and fp8 scales are: a few bytes
+//    per tile, whose loads the sums' way through LDS mostly covers);
 //  - no kernel reads the batch's row count first: every row of the launch is
 //    computed (the buffers hold them), whatever is in the surplus ones (but for a
 //    residual stream in the caller's memory, whose rows end with the batch);
@@ -18,8 +19,9 @@
 //
 // Measured per launch at 128 rows of a 768-wide layer (start to start in a
 // replayed graph, against the 64x32 and split-K tiles these replace there): QKV
-// + RoPE 8.0 -> 5.4 us, Wi + GEGLU 7.9 -> 5.0, Wo2 with the LayerNorm after it
-// 10.9 -> 8.0; at 256 rows 8.2 -> 8.4, 8.2 -> 7.4 and 12.3 -> 10.1.  At 640 rows
+// + RoPE 8.0 -> 5.1 us (5.4 while its tables waited for the operands), Wi + GEGLU
+// 7.9 -> 5.0, Wo2 with the LayerNorm after it 10.9 -> 8.0; at 256 rows Wo2 12.3 ->
+// 10.1, QKV 8.2 -> 7.8, Wi 8.2 -> 7.4.  At 640 rows
 // the 64x64 tiles are the faster ones (10.6 against 11.9, 10.9 against 11.3).
 // With fp8 weights, which had one 256x256 tile shape, four layers of 128 rows
 // take 175 us and 256 rows 224 us, against 636.  The LayerNorm before a product
@@ -99,10 +101,22 @@ __global__ __launch_bounds__(256) void gemm_short_kernel(GemmArgs g) {
   // epilogue items: two neighbouring columns (of a pair's lower half) each
   constexpr int EC = EPI == EPI_STORE ? BN / 2 : BN / 4, ES = BM * EC / 256;
   static_assert(BM * EC % 256 == 0, "epilogue items");
+  // A RoPE tile's positions come through the scalar cache, eight rows per wave, so
+  // that the table loads wait for them and for no operand (a vector load's wait
+  // would drain those issued after it as well).
   int pos[ES];
   if constexpr (EPI == EPI_ROPE) {
+    static_assert(EC == 8, "eight rows of items per wave");
 #pragma unroll
-    for (int s = 0; s < ES; ++s) pos[s] = g.pos[m0 + (tid + 256 * s) / EC];
+    for (int s = 0; s < ES; ++s) {
+      const int* pr = g.pos + m0 + 32 * s + 8 * wave;  // uniform
+      pos[s] = __builtin_amdgcn_readfirstlane(pr[0]);
+#pragma unroll
+      for (int i = 1; i < 8; ++i) {
+        const int p = __builtin_amdgcn_readfirstlane(pr[i]);  // (else the selected address is loaded, by lane)
+        pos[s] = (lane >> 3) == i ? p : pos[s];
+      }
+    }
   }
 
   // operand loads: instruction j of a stage moves 1 KB, 8 rows of 128 bytes (16
@@ -134,7 +148,6 @@ __global__ __launch_bounds__(256) void gemm_short_kernel(GemmArgs g) {
   for (int grp = 0; grp < R; ++grp) issue_group(grp);
   __builtin_amdgcn_sched_barrier(0);
   f32x2_t cs[ES], sn[ES];
-  constexpr int EXTRA = EPI == EPI_ROPE ? 2 * ES : 0;  // loads issued after the first R groups
   if constexpr (EPI == EPI_ROPE) {
 #pragma unroll
     for (int s = 0; s < ES; ++s) {
@@ -155,12 +168,12 @@ __global__ __launch_bounds__(256) void gemm_short_kernel(GemmArgs g) {
   for (int t = 0; t < TI; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto step = [&](auto grp_tag) {
     constexpr int grp = decltype(grp_tag)::value;
-    // loads of this wave issued after group grp's: later groups of the first R,
-    // the epilogue's, and the refills so far (one per group consumed)
+    // operand loads of this wave issued after group grp's: the later groups of the
+    // first R and the refills so far (one per group consumed).  The table loads are
+    // not counted: how many the compiler makes of them, and where it puts them,
+    // must not decide whether a group has landed.
     constexpr int last = grp - 1 + R < NG - 1 ? grp - 1 + R : NG - 1;
-    constexpr int after = grp < R ? (R - 1 - grp) * T::PER_GROUP + EXTRA + (last - (R - 1)) * T::PER_GROUP
-                                  : (last - grp) * T::PER_GROUP;
-    wait_vmcnt<after>();
+    wait_vmcnt<(last - grp) * T::PER_GROUP>();
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int s = 0; s < GR; ++s) {
