@@ -21,7 +21,7 @@
 // replayed graph, against the 64x32 and split-K tiles these replace there): QKV
 // + RoPE 8.0 -> 5.1 us (5.4 while its tables waited for the operands), Wi + GEGLU
 // 7.9 -> 5.0, Wo2 with the LayerNorm after it 10.9 -> 8.0; at 256 rows Wo2 12.3 ->
-// 10.1, QKV 8.2 -> 7.8, Wi 8.2 -> 7.4.  At 640 rows
+// 10.1 (the others: plain_pays).  At 640 rows
 // the 64x64 tiles are the faster ones (10.6 against 11.9, 10.9 against 11.3).
 // With fp8 weights, which had one 256x256 tile shape, four layers of 128 rows
 // take 175 us and 256 rows 224 us, against 636.  The LayerNorm before a product
@@ -294,13 +294,31 @@ void launch_k(const GemmArgs& g, hipStream_t st) {
   }
 }
 
+int plain_tiles(const GemmArgs& g) {
+  return (g.epi == EPI_GEGLU ? (g.N + 15) / 16 : (g.N + 31) / 32) * (g.M / 32);
+}
+
+// How many tiles these kernels take of a product, by whole layers in replayed graphs
+// against the 64x32 tiles (fp8: 64x64): all that run at once, two per CU (192 rows of
+// a 768-wide layer, 432 tiles: QKV 2.3 us less, Wi + GEGLU 2.2). A second round
+// saves less (Wi + GEGLU of 192 rows at K = 1024, 984 tiles: 0.5, with fp8 weights
+// 0.6), and loses where the third begins (256 rows, 1312 tiles: 0.4 and 1.4 more).
+// It loses at once for biased products (the decision head's at 256 rows, 576 and 768
+// tiles: ~1.5 more) and QKV at K up to 768 (256 rows, 576 tiles: 0.6 more; at K =
+// 1024, 768 tiles, 1.3 less, with fp8 weights 2.1-2.5 less).  Wi + GEGLU of the same
+// 256 rows at K = 768 gains 0.5 on the other tiles while QKV stays here, but both
+// there lose 1.2, so that one of the two goes.
+bool plain_pays(const GemmArgs& g) {
+  const bool one_round = g.epi == EPI_STORE || (g.epi == EPI_ROPE && g.K <= 768 && g.w_dtype != DT_FP8);
+  return plain_tiles(g) <= (one_round ? 2 : 4) * num_cus();
+}
+
 template <bool W8>
 void launch_plain(const GemmArgs& g, hipStream_t st) {
   // the whole K in flight (96 KB of LDS at K = 768) while every tile has a CU of
   // its own; else half the ring, so that two tiles share a CU (128 rows, 288
   // tiles: QKV 5.4 us, against 6.3 with 64-row tiles of the whole K)
-  const int tiles_n = g.epi == EPI_GEGLU ? (g.N + 15) / 16 : (g.N + 31) / 32;
-  if (tiles_n * (g.M / 32) <= num_cus())
+  if (plain_tiles(g) <= num_cus())
     launch_k<32, 4, W8>(g, st);
   else
     launch_k<32, 2, W8>(g, st);
@@ -457,9 +475,8 @@ bool gemm_short_ok(const GemmArgs& g) {
     return false;
   if (g.epi == EPI_ROPE)
     return g.head_dim == 64 && g.N % 64 == 0 && g.rope_dim % 64 == 0 && g.pos && g.rope_cos && g.rope_sin &&
-           aligned(g.rope_cos, 8) && aligned(g.rope_sin, 8) && g.rope_rows > 0 && 2 * g.rope_dim <= g.N;
-  if (g.epi == EPI_GEGLU) return g.N % 16 == 0;
-  return g.epi == EPI_STORE;
+           aligned(g.rope_cos, 8) && aligned(g.rope_sin, 8) && g.rope_rows > 0 && 2 * g.rope_dim <= g.N && plain_pays(g);
+  return (g.epi == EPI_STORE || (g.epi == EPI_GEGLU && g.N % 16 == 0)) && plain_pays(g);
 }
 
 void launch_gemm_short(const GemmArgs& g, hipStream_t st) {

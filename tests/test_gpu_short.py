@@ -55,6 +55,14 @@ def test_short_fp8_rows(orc, D, lens):
     om = orc.model(sj.fp8_dequantized(w), cfg)
     h, ref = m.encode(ids, mask), om.encode(ids, mask)
     assert float(np.abs(h - ref)[mask.astype(bool)].max()) <= 2e-2
+    # the same bits in a batch that fills the range, where the products of more than
+    # two rounds of tiles go to the tiled kernels
+    if sum(lens) < 256:
+        fids, fmask, _ = synth.batch_with_lens(lens + [256 - sum(lens)], 256 - sum(lens), 1024, seed=6)
+        fids[:len(lens), :ids.shape[1]] = ids
+        full = m.encode(fids, fmask)
+        for b, k in enumerate(lens):
+            assert np.array_equal(h[b, :k], full[b, :k]), f"row {b}"
     mp, mm, qt = synth.make_markers(n, 4, [(0, 4), (2, 2)][:len(lens)], seed=7)
     logits, act = m.forward(ids, mask, mp, mm, qt)
     rl, ra = om.forward(ids, mask, mp, mm, qt)
