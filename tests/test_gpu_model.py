@@ -42,6 +42,16 @@ def probs_err(orc, lg, lr, mm):
     return e
 
 
+def launched(ids, mask, w, cfg, **kw):
+    """Names of the launches of one encode (profiled, launch by launch)."""
+    m = sj.Model(w, cfg, precision=BF16, **kw)
+    m.profile(True)
+    m.encode(ids, mask)
+    names = set(m.profile_read())
+    m.close()
+    return names
+
+
 def labels(orc, lg, mm):
     return [int(np.argmax(orc.calibrated_probs(lg[b, :int(mm[b].sum())], 1.0))) for b in range(len(lg))]
 
@@ -242,8 +252,8 @@ def test_folded_layer_norm_under_large_row_offsets(orc, offset):
 
 @pytest.mark.parametrize("offset", ["none", "row", "block"])
 def test_residual_epilogue_layer_norm(orc, offset):
-    # On one round of persistent 256 x 256 tiles (T >= 4096, at most 256
-    # tiles) the residual GEMMs' epilogues also write the LayerNorm that reads
+    # On one round of persistent 256 x 256 tiles (128 to 256 of them on 256
+    # CUs) the residual GEMMs' epilogues also write the LayerNorm that reads
     # the residual stream next: the tiles of a 256-row panel publish their
     # rows' 256-column moments and each normalises its own block once the
     # panel's other tiles have arrived.  Checked against the standalone
@@ -267,10 +277,11 @@ def test_residual_epilogue_layer_norm(orc, offset):
         for i in range(cfg["num_hidden_layers"]):
             k = f"encoder.layers.{i}.mlp.Wo.weight"
             w[k] = synth.bf16_round(w[k] + np.outer(v, u).astype(np.float32) / np.sqrt(F))
-    ids, mask, lens = synth.make_batch(12, 480, 380, 480, cfg["vocab_size"], seed=28)
+    ids, mask, lens = synth.make_batch(27, 480, 400, 480, cfg["vocab_size"], seed=28)
     T = int(lens.sum())
-    assert 4096 <= T and 3 * ((T + 255) // 256) <= 256
+    assert 128 <= 3 * ((T + 255) // 256) <= 256
     print(f"rln {offset}: T={T}", flush=True)
+    assert {"gemm_wo_resid_ln", "gemm_wo2_resid_ln"} <= launched(ids, mask, w, cfg)
     fused = sj.Model(w, cfg, precision=BF16)
     h1 = fused.encode(ids, mask)
     h2 = fused.encode(ids, mask)
@@ -318,10 +329,11 @@ def test_residual_epilogue_layer_norm_widths(orc, D, H, F):
     for k in list(w):
         if k.endswith(("attn_norm.weight", "mlp_norm.weight")):
             w[k] = synth.bf16_round((1.0 + 0.2 * rng.standard_normal(D)).astype(np.float32))
-    ids, mask, lens = synth.make_batch(12, 480, 380, 480, cfg["vocab_size"], seed=73)
+    ids, mask, lens = synth.make_batch(20 * 1024 // D, 480, 400, 480, cfg["vocab_size"], seed=73)
     T = int(lens.sum())
-    assert 4096 <= T and (D // 256) * ((T + 255) // 256) <= 256
+    assert 128 <= (D // 256) * ((T + 255) // 256) <= 256
     print(f"rln D={D}: T={T}", flush=True)
+    assert {"gemm_wo_resid_ln", "gemm_wo2_resid_ln"} <= launched(ids, mask, w, cfg)
     fused = sj.Model(w, cfg, precision=BF16)
     h1 = fused.encode(ids, mask)
     fused.close()
@@ -511,22 +523,23 @@ def test_graph_replay_serves_a_shape_bucket():
 
 
 def test_graph_replay_with_residual_epilogue_layer_norm():
-    # Batches of one shape bucket at T > 4096 (one round of persistent
-    # residual tiles, whose epilogue finishes the LayerNorm through the row
-    # panels' sync ints) replay one captured graph: every launch leaves the
-    # ints at zero for the next replay.  Each result equals the launch-by-
-    # launch run with the standalone LayerNorm, bit for bit.
+    # Batches of one shape bucket whose residual products take one round of
+    # persistent tiles (at 12 288 launched rows 144 of them), whose epilogue
+    # finishes the LayerNorm through the row panels' sync ints, replay one
+    # captured graph: every launch leaves the ints at zero for the next replay.
+    # Each result equals the launch-by-launch run with the standalone LayerNorm,
+    # bit for bit.
     rl, enc, w = synth.make_model(**dict(synth.PRESETS["cfg2"], num_hidden_layers=2), seed=48)
     cfg = synth.flat_cfg(rl, enc)
     g_on = sj.Model(w, cfg, precision=BF16, use_graphs=True)
     g_off = sj.Model(w, cfg, precision=BF16, use_graphs=False, fuse_ln=0)
     V = cfg["vocab_size"]
-    batches = [synth.batch_with_lens([370, 380, 360, 375, 365, 384, 372, 368, 377, 366, 371, 369], 384, V, seed=49),
-               synth.batch_with_lens([384, 300, 380, 350, 383, 376, 379, 381, 382, 330, 378, 380, 10], 384, V,
-                                     seed=50),
-               synth.batch_with_lens([350, 360, 340, 370, 345, 355, 365, 380, 384, 375, 362, 358], 384, V, seed=51)]
+    rng = np.random.default_rng(49)
+    batches = [synth.batch_with_lens([*rng.integers(lo, 385, size=n - 1), last], 384, V, seed=49 + n)
+               for n, lo, last in ((32, 355, 384), (32, 366, 10), (31, 376, 300))]
     for ids, mask, lens in batches:
-        assert 4096 < int(lens.sum()) <= 4608 and 256 < lens.max() <= 384
+        assert 11264 < int(lens.sum()) <= 12288 and 256 < lens.max() <= 384 and len(lens) <= 32
+    assert {"gemm_wo_resid_ln", "gemm_wo2_resid_ln"} <= launched(*batches[1][:2], w, cfg)
     for i, (ids, mask, lens) in enumerate(batches + [batches[0]]):
         h = g_on.encode(ids, mask)
         want = g_off.encode(ids, mask)
