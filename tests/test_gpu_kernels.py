@@ -52,13 +52,15 @@ def rnd(rng, shape, scale=1.0):
     return bf16_round((rng.standard_normal(shape) * scale).astype(np.float32))
 
 
-# (4500, 512, 64) and (4200, 256, 128) take the persistent kernel (M >= 4096)
-# with fewer K steps per tile than its load ring keeps in flight: the ring then
-# moves on to the next tile during the prologue (regression case)
+# (20500, 512, 64) and (41000, 256, 128) take the persistent kernel (more than 160
+# tiles on 256 CUs) with fewer K steps per tile than its load ring keeps in flight:
+# the ring then moves on to the next tile during the prologue (regression case);
+# (4500, 512, 64) and (4200, 256, 128): the same on the 128x128 and 128x64 tiles
 # (130, 200, 128) and (600, 200, 128): a last column tile past N on the 64x32
 # and 64x64 tiles (the store epilogue's bounds-checked body)
 @pytest.mark.parametrize("M,N,K", [(300, 256, 128), (1, 128, 64), (130, 384, 192), (640, 2304, 768),
-                                   (4500, 512, 64), (4200, 256, 128), (130, 200, 128), (600, 200, 128)])
+                                   (4500, 512, 64), (4200, 256, 128), (130, 200, 128), (600, 200, 128),
+                                   (20500, 512, 64), (41000, 256, 128)])
 @pytest.mark.parametrize("act", [0, 1, 2])
 def test_gemm_bf16_mfma(orc, M, N, K, act):
     print(f"gemm bf16 M={M} N={N} K={K} act={act}", flush=True)
@@ -371,16 +373,20 @@ def test_gemm_persistent_half_units(orc, kind):
         assert rel_err(host(O), want) < 8e-3
 
 
+@pytest.mark.parametrize("M", [20600, 4500])
 @pytest.mark.parametrize("kind", ["store", "resid", "geglu", "rope"])
-def test_gemm_persistent_ragged_columns(orc, kind):
-    # persistent kernel (M >= 4096) whose last row tile runs past M and whose
-    # last column tile runs past N: the epilogues' bounds-checked instantiation
-    # next to the bounds-free one; three K steps, so RoPE tables are copied
-    # during the last K step
-    M, K, H, Dh, L = 4500, 192, 5, 64, 700
+def test_gemm_persistent_ragged_columns(orc, kind, M):
+    # persistent kernel (M 20600: 162 tiles or more; 4500 rows take the tiled
+    # ones) whose last row tile runs past M and whose last column tile runs past
+    # N: the epilogues' bounds-checked instantiation next to the bounds-free one;
+    # three K steps, so RoPE tables are copied during the last K step
+    K, H, Dh, L = 192, 5, 64, 700
     n = {"store": 320, "resid": 320, "geglu": 320, "rope": 3 * H * Dh}[kind]
     nw = 2 * n if kind == "geglu" else n
-    print(f"persistent ragged columns: {kind} M={M} N={n} K={K}", flush=True)
+    tiles = -(-n // (128 if kind == "geglu" else 256)) * -(-M // 256)
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    print(f"persistent ragged columns: {kind} M={M} N={n} K={K} tiles={tiles}", flush=True)
+    assert (8 * tiles >= 5 * ncu) == (M == 20600)
     rng = np.random.default_rng(91)
     a, w, b = rnd(rng, (M, K)), rnd(rng, (nw, K), 0.1), rnd(rng, n)
     A, W = dev(a, torch.bfloat16), dev(w, torch.bfloat16)
@@ -410,11 +416,12 @@ def test_gemm_persistent_ragged_columns(orc, kind):
 
 
 def test_gemm_tile_shape_invariance():
-    # the tile shape is chosen from M; a row's result must not depend on it
+    # the tile shape follows the number of tiles (at 11 000 rows 128x128 tiles
+    # would need a second round); a row's result must not depend on it
     # (bit-identical for every epilogue)
     rng = np.random.default_rng(5)
     K, H, Dh, L = 768, 12, 64, 512
-    Mb, Ms = 5000, 200
+    Mb, Ms = 11000, 200
     a = rnd(rng, (Mb, K))
     A = dev(a, torch.bfloat16)
     c, s = (np.cos(np.arange(L * 32).reshape(L, 32) * 1e-3).astype(np.float32),
@@ -425,7 +432,7 @@ def test_gemm_tile_shape_invariance():
                         ("rope", 2304, 2304)):
         W = dev(rnd(rng, (nw, K), 0.05), torch.bfloat16)
         res = []
-        for M in (Mb, 1500, 300, Ms):  # persistent, 128x128, 64x64 and (GEGLU, store, RoPE) 64x32 tiles
+        for M in (Mb, 5000, 1500, 300, Ms):  # persistent, 128x128, smaller and (GEGLU, store, RoPE) 64x32 tiles
             odt = torch.float32 if kind == "resid" else torch.bfloat16
             O = torch.zeros((M, n), dtype=odt, device="cuda")
             if kind == "store":
