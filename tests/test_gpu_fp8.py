@@ -81,6 +81,33 @@ def test_gemm_fp8w_vs_dequantized_fp32(M, N, K, act, bias):
     assert err <= 1e-2
 
 
+@pytest.mark.parametrize("D,H,F", [(768, 12, 1152), (1024, 16, 2624)])
+def test_fp8_rows_keep_their_bits_at_every_tile_shape(orc, D, H, F):
+    # batches whose projections take each tile shape (64x64 to the persistent
+    # kernel), through RoPE, GEGLU and residual epilogues: a sequence's hidden
+    # states keep their bits from one to the next, and the oracle on the
+    # dequantized weights holds them
+    rl, enc, w = synth.make_model(hidden_size=D, num_hidden_layers=2, num_attention_heads=H, intermediate_size=F,
+                                  vocab_size=1024, theta_full=160000.0, store="BF16", seed=57)
+    cfg = synth.flat_cfg(rl, enc)
+    m = sj.Model(w, cfg, precision=sj.SJH_PREC_FP8W)
+    n = 121
+    ids0 = np.random.default_rng(58).integers(0, 1024, size=n)
+    first = None
+    for total in (300, 641, 1500, 2304, 4000, 5000, 11000):
+        lens = [n] + [400] * ((total - n) // 400)
+        lens += [total - sum(lens)] if total > sum(lens) else []
+        ids, mask, _ = synth.batch_with_lens(lens, max(lens), 1024, seed=total)
+        ids[0, :n] = ids0
+        print(f"fp8 rows D={D} T={total}", flush=True)
+        h = m.encode(ids, mask)[0, :n]
+        first = h if first is None else first
+        assert np.array_equal(h, first), total
+    m.close()
+    ref = orc.model(sj.fp8_dequantized(w), cfg).encode(ids0[None], np.ones((1, n), np.int64))[0]
+    assert float(np.abs(first - ref).max()) <= 2e-2
+
+
 def test_cfg5_shape_model_vs_reference_on_dequantized_weights(orc):
     # BASELINE config 5's encoder widths (D=1024, 16 heads, GEGLU 2624, V=50368)
     # through 2 layers: encode of two sequences, and the decision head on one
