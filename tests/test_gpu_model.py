@@ -630,6 +630,42 @@ def test_calls_on_two_streams_and_forward_are_ordered():
     m.close()
 
 
+@pytest.mark.parametrize("graphs", [True, False])
+def test_null_stream_and_named_streams_are_ordered(graphs):
+    # Calls that alternate between the legacy null stream and named ones (which
+    # do not wait for it by themselves), with and without graphs, among them
+    # allocation-free calls, share the workspace or the fixed array: each waits
+    # for the call before.  No host synchronization between them; every result
+    # equals the same call made alone.
+    import torch
+
+    rl, enc, w = synth.make_model(**dict(synth.PRESETS["cfg2"], num_hidden_layers=2), seed=51)
+    cfg = synth.flat_cfg(rl, enc)
+    m = sj.Model(w, cfg, precision=BF16, use_graphs=graphs)
+    D = cfg["hidden_size"]
+    d_ids, d_out, want, all_lens = [], [], [], []
+    for i, n in enumerate((1500, 90, 700, 200, 1900, 60)):
+        lens = np.array([n // 2, n - n // 2], np.int32)
+        ids, mask, _ = synth.batch_with_lens(list(lens), int(lens.max()), cfg["vocab_size"], seed=62 + i)
+        h = m.encode(ids, mask)
+        want.append(np.concatenate([h[b, :lens[b]] for b in range(2)]))
+        d_ids.append(torch.from_numpy(np.concatenate([ids[b, :lens[b]] for b in range(2)]).astype(np.int32)).cuda())
+        d_out.append(torch.full((n, D), float("nan"), dtype=torch.float32, device="cuda"))
+        all_lens.append(lens)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()  # default priority
+    torch.cuda.synchronize()
+    for rep in range(3):  # the first captures, the others replay
+        for i, st in enumerate((0, a.cuda_stream, 0, b.cuda_stream, a.cuda_stream, 0)):
+            fn = m.encode_device_noalloc if (i + rep) % 3 == 2 else m.encode_device
+            fn(d_ids[i].data_ptr(), all_lens[i], d_out[i].data_ptr(), st)
+        torch.cuda.synchronize()
+        for i in range(len(want)):
+            assert np.array_equal(d_out[i].cpu().numpy(), want[i]), (rep, i)
+            d_out[i].fill_(float("nan"))
+        torch.cuda.synchronize()
+    m.close()
+
+
 @pytest.mark.parametrize("prec", [FP32, BF16])
 def test_hidden_wider_than_1024_at_batch_one(orc, prec):
     # D = 1536: the layer norms take the scalar row kernel, so the short
