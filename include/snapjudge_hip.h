@@ -107,9 +107,9 @@ typedef struct sjh_options {
                          only on valid tokens (padded positions of encode() are 0) */
   int32_t device;     /* HIP device ordinal */
   int32_t fuse_ln;    /* 1 (default): where a residual GEMM's tiles all run at once (bf16,
-                         hidden size a multiple of 256 up to 1024, one round of at least
-                         128 tiles), its epilogue also writes the LayerNorm that reads the
-                         residual stream next; 0: that LayerNorm runs as a launch of its
+                         hidden size a multiple of 256 up to 1024, one round of tiles on
+                         at least half the CUs), its epilogue also writes the LayerNorm
+                         that reads the residual stream next; 0: that LayerNorm runs as a launch of its
                          own; 2: as 1 with any number of tiles, and a tile waits for its
                          panel's other tiles for one poll only, so that most tiles take
                          the path of a tile that gave up waiting (the results are the

@@ -1931,7 +1931,9 @@ bool pers_ok(const GemmArgs& g) {
 // What bounds these products between the latency of a few rows and the matrix
 // pipes of a full chip is each CU's intake: ~50 GB/s from L2 into LDS however
 // many stages are in flight, so a product wants its tiles on every CU, then
-// tiles as large as that leaves (fewer bytes per output).  Per launch, us, M x
+// tiles as large as that leaves (fewer bytes per output).  T128's 12 steps at K =
+// 768, one stage in flight, rather wait for each stage's loads (1501 x 3072 x 768
+// took as long on 192x128 tiles, with 62% of the bytes per CU).  Per launch, us, M x
 // N x K, on the shapes' neighbours (bench of every shape at 320 to 18 432 rows):
 //  T64     64x64, 2 waves, 4 stages, up to a tile per CU: 1024 x 768 x 1152 9.9
 //          (128x64 10.7, 128x128 12.3)

@@ -33,7 +33,9 @@
 // of two v_mfma_f32_32x32x16_bf16 over the same k values (the same bits on the
 // device over 24 chained steps of random values), so a product here has the
 // bits of the other bf16 kernels': sum over K in order for plain, RoPE and
-// GEGLU products; for residual ones the K slices of split_k_slices().
+// GEGLU products; for residual ones the K slices of split_k_slices().  With fp8
+// weights the residual products of more rows sum K in one chain, so that a row's
+// bits differ between batches of up to 256 rows and larger ones, as bf16 rows' do.
 #include <algorithm>
 #include <type_traits>
 
